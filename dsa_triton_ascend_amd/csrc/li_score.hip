@@ -412,6 +412,217 @@ __global__ __launch_bounds__(NW * 64) void li_score_kernel(LiScoreArgs a) {
   wait_vmcnt<0>();   // no direct-to-LDS load may outlive the work-group's LDS
 }
 
+// ---------------------------------------------------------------- few query rows (decode)
+// Batches of at most ROWS_MAX query rows (a decode step, with speculative tokens a few): the
+// call reads every key once for one or a few rows, so it is bound by HBM (256 bytes a key against
+// 32 MFMA cycles), and the kernel above keeps one of its eight waves busy there. Here a
+// work-group (four waves) takes `chunk` keys of one row and its waves take the chunk's 32-key
+// subtiles in turn, each on its own: a wave copies a subtile (8 KB) into one of its two LDS
+// buffers while it computes the one before, so no barrier couples the waves and eight waves keep
+// 64 KB a CU in flight. The Q fragments (G <= 64) stay in VGPRs. Chunks are cut from the row's
+// own visible length, so sequences of uneven lengths leave no work-group with a long one; the
+// rows of one batch are dispatched 8 work-groups apart, on one XCD, whose L2 then serves the
+// second row's keys, and the chunk an XCD starts with turns with the batch (the last chunks of
+// short sequences are empty: without the turn the XCDs that take them idle, 48 -> 38 us for 200
+// sequences of 300 .. 6000 tokens). Same products, sums and rounding order as above.
+// 64 sequences of 4K .. 32K tokens (302 MB of keys), against the kernel above: 118 -> 60.5 us
+// (5.0 TB/s; a large copy moves 4.9). The rows of one batch share no registers, so their cost adds
+// up: 2 rows each 125 -> 96 us, 3 rows 134 -> 110, 4 rows 144 -> 130; from 5 on the kernel above.
+constexpr int ROWS_MAX = 4;
+constexpr int ROWS_NW = 4;            // waves per work-group
+constexpr int ROWS_CHUNK_MAX = 2048;  // keys per work-group
+
+template <int IO, int MT, bool PAGED>
+__global__ __launch_bounds__(ROWS_NW * 64, 2) void li_score_rows_kernel(LiScoreArgs a, int chunk, int nchunk) {
+  constexpr int D = 128, KK = D / 16, SUB = 32, NT = ROWS_NW * 64;
+  __shared__ __attribute__((aligned(16))) uint16_t kt[ROWS_NW][2][SUB * D];
+  __shared__ int bt_s[PAGED ? ROWS_CHUNK_MAX + 1 : 1];   // first cache row of the chunk's pages, -1: missing
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.z, n2 = blockIdx.y;
+  // blockIdx.x = (group of 8 chunks, row, chunk of the group)
+  const int R = a.max_rows_per_batch;
+  const int x8 = (int)blockIdx.x >> 3;
+  const int ch = (x8 / R) * 8 + (((int)blockIdx.x + b) & 7), s1 = x8 % R;
+  const int rows_b = a.row_start[b + 1] - a.row_start[b];
+  const int aq = a.act_q[b], ak = a.act_k[b];
+  if (ch >= nchunk || s1 >= rows_b || s1 >= aq) return;
+  const int L = visible_len(s1, aq, ak, a.s2, a.sparse_mode);
+  int c0 = ch * chunk;
+  if (c0 >= L) return;
+  const int G = a.n1 / a.n2;
+  const int64_t r = (int64_t)a.row_start[b] + s1;
+  const uint16_t* qrow = reinterpret_cast<const uint16_t*>(a.q) + (r * a.n1 + (int64_t)n2 * G) * D;
+  const char* kbase = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.k) +
+                                                    ((PAGED ? 0 : (int64_t)a.key_start[b]) * a.n2 + n2) * D);
+  const uint32_t ksb = (uint32_t)(a.n2 * D * 2);   // key row stride in bytes
+  const int page = PAGED ? a.page_bs : 1;
+  const int pshift = PAGED && (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1;
+  auto block_of = [&](int t) { return pshift >= 0 ? t >> pshift : t / page; };
+  // pages of whole 32-key subtiles, all of them inside the cache: a subtile is 32 cache rows
+  const bool whole = PAGED && page % SUB == 0 && a.key_rows % page == 0;
+  int b0 = 0;   // first block-table entry of the chunk
+  auto bt_load = [&](int i) -> int {
+    return b0 + i < a.max_blocks ? a.block_table[(int64_t)b * a.max_blocks + b0 + i] : -1;
+  };
+  // (a cache of 256-byte rows in device memory holds fewer than 2^31 of them)
+  auto page_row = [&](int blk) { return blk >= 0 && (int64_t)blk * page < a.key_rows ? blk * page : -1; };
+  // cache row of key t (row 0 for a missing block: its scores are written as 0)
+  const uint32_t krows = PAGED ? (uint32_t)a.key_rows : 0u;
+  auto phys_row = [&](int t, bool& ok) -> uint32_t {
+    const int bi = block_of(t);
+    const int base = bt_s[bi - b0];
+    const uint32_t p = (uint32_t)base + (uint32_t)(t - bi * page);
+    ok = base >= 0 && p < krows;
+    return ok ? p : 0u;
+  };
+  // Copy j of a subtile fills its key rows 4j .. 4j + 3 (16 lanes a row); chunk c of key row k sits
+  // at c ^ (k & 15). Keys past the last visible one re-read it (or, in a whole page, that page's
+  // rows); their columns are never stored.
+  uint32_t voff[SUB / 4];
+#pragma unroll
+  for (int j = 0; j < SUB / 4; ++j) {
+    const int k = 4 * j + (lane >> 4);
+    voff[j] = (uint32_t)k * ksb + 16u * (uint32_t)((lane & 15) ^ (k & 15));
+  }
+  auto dma = [&](int t0, uint16_t* buf) __attribute__((always_inline)) {
+    if (PAGED ? whole : t0 + SUB <= L) {
+      uint32_t row = (uint32_t)t0;
+      if constexpr (PAGED) {
+        bool ok;
+        row = phys_row(t0, ok);
+      }
+      const uint64_t u = reinterpret_cast<uint64_t>(kbase + (uint64_t)row * ksb);   // wave-uniform
+      const char* base = reinterpret_cast<const char*>(
+          ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) |
+          (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u));
+#pragma unroll
+      for (int j = 0; j < SUB / 4; ++j) lds_dma16_sbase_untracked(base, voff[j], buf + j * 512);
+    } else {
+#pragma unroll
+      for (int j = 0; j < SUB / 4; ++j) {
+        const int k = 4 * j + (lane >> 4);
+        const int t = t0 + k < L ? t0 + k : L - 1;
+        uint32_t row = (uint32_t)t;
+        if constexpr (PAGED) {
+          bool ok;
+          row = phys_row(t, ok);
+        }
+        lds_dma16_untracked(kbase + (uint64_t)row * ksb + 16 * ((lane & 15) ^ (k & 15)), buf + j * 512);
+      }
+    }
+  };
+
+  // the first chunk's block-table entries are requested ahead of Q and the weights
+  int bt_first = -1;
+  if constexpr (PAGED) {
+    b0 = block_of(c0);
+    bt_first = bt_load(threadIdx.x);
+  }
+  uint4 qf[MT][KK];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = mt * 32 + (lane & 31);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) qf[mt][kk] = ldg16_or0(m < G, qrow + (int64_t)m * D + kk * 16 + (lane >> 5) * 8);
+  }
+  const float wl = lane < G ? load_w(a.w, a.wdt, r * a.n1 + (int64_t)n2 * G + lane) : 0.f;
+  asm volatile("" ::: "memory");
+  const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc(
+      a.scores + (r * a.n2 + n2) * a.ld, (short)0, L * 2, 0x00020000);
+
+  uint16_t* const buf0 = kt[wave][0];
+  // fragment of a buffer: key lane % 32, chunk 2 kk + lane / 32
+  const uint16_t* rp[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) rp[kk] = buf0 + (lane & 31) * D + 8 * ((2 * kk + (lane >> 5)) ^ (lane & 15));
+  float wv[MT][16];
+  bool first = true;
+  // one chunk, unless the row is longer than the max_kv that sized the grid
+  for (;; c0 += nchunk * chunk) {
+    const int c1 = c0 + chunk < L ? c0 + chunk : L;   // the chunk's visible keys end here
+    const int nsub = (c1 - c0 + SUB - 1) / SUB;
+    if constexpr (PAGED) {
+      if (!first) lds_barrier();   // every wave is done with the last chunk's entries
+      b0 = block_of(c0);
+      const int nb = block_of(c1 - 1) - b0 + 1;
+      for (int i = threadIdx.x; i < nb; i += NT) bt_s[i] = page_row(first && i < NT ? bt_first : bt_load(i));
+      lds_barrier();
+    }
+    int bufi = 0;
+    if (wave < nsub) dma(c0 + wave * SUB, buf0);
+    if (first) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) wv[mt][i] = __shfl(wl, mt * 32 + m32_row(i, lane));
+      first = false;
+    }
+    // the score of the last subtile is stored after the next one's copies are issued and waited
+    // for, so no store sits ahead of the copies that a wait retires
+    float prev = 0.f;
+    int prev_key = -1;
+    auto store = [&]() __attribute__((always_inline)) {
+      if (prev_key >= 0 && lane < 32) {
+        float v = prev;
+        const int t = prev_key + lane;
+        if constexpr (PAGED) {
+          bool ok;
+          phys_row(t < L ? t : L - 1, ok);
+          v = ok ? v : 0.f;
+        }
+        __builtin_amdgcn_raw_buffer_store_b16(from_f32<IO>(v), srd, t * 2, 0, 0);
+      }
+    };
+    for (int sub = wave; sub < nsub; sub += ROWS_NW) {
+      // the other buffer's fragment reads (the subtile before) have returned: it can be overwritten
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (sub + ROWS_NW < nsub) {   // wave-uniform
+        dma(c0 + (sub + ROWS_NW) * SUB, buf0 + (bufi ^ 1) * SUB * D);
+        wait_vmcnt<SUB / 4>();   // everything before these copies, so this subtile, has landed
+      } else {
+        wait_vmcnt<0>();
+      }
+      asm volatile("" ::: "memory");
+      store();
+      uint4 bf[KK];
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) bf[kk] = *reinterpret_cast<const uint4*>(rp[kk] + bufi * SUB * D);
+      f32x16 acc[MT];
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt] = Mfma<IO>::m32(qf[mt][kk], bf[kk], kk == 0 ? f32x16{} : acc[mt]);
+      float p4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < MT * 16; ++e) p4[e & 3] += fmaxf(acc[e >> 4][e & 15], 0.f) * wv[e >> 4][e & 15];
+      prev = add_half_swap((p4[0] + p4[1]) + (p4[2] + p4[3]));
+      prev_key = c0 + sub * SUB;
+      bufi ^= 1;
+    }
+    store();
+    if (L - c0 <= nchunk * chunk) break;
+  }
+}
+
+template <int IO, bool PAGED>
+void launch_rows(const LiScoreArgs& a, hipStream_t s, int MT) {
+  // keys per work-group: the largest of 256 .. 2048 with at least 384 work-groups at the longest
+  // length (the others are shorter by an unknown share, and a CU holds two). Fewer, longer ones
+  // spare Q loads and prologues: 64 sequences of 4K .. 32K, 2048 keys 60.5 us, 1024 67, 512 72;
+  // 200 of 300 .. 6000, 2048 39, 512 49; 8 of 3K .. 60K, 1024 16.9, 512 19.7, 256 22; one of
+  // 100000, 256 9.0, 128 13.1.
+  const int64_t rows = (int64_t)a.max_rows_per_batch * a.n2 * a.batch;
+  const int kv = a.max_kv > 0 ? a.max_kv : 1;
+  int chunk = ROWS_CHUNK_MAX;
+  while (chunk > 256 && rows * ((kv + chunk - 1) / chunk) < 384) chunk >>= 1;
+  const int nchunk = (kv + chunk - 1) / chunk;
+  const dim3 grid((unsigned)((nchunk + 7) / 8 * 8 * a.max_rows_per_batch), a.n2, a.batch), block(ROWS_NW * 64);
+  if (MT == 1) hipLaunchKernelGGL((li_score_rows_kernel<IO, 1, PAGED>), grid, block, 0, s, a, chunk, nchunk);
+  else hipLaunchKernelGGL((li_score_rows_kernel<IO, 2, PAGED>), grid, block, 0, s, a, chunk, nchunk);
+}
+
 template <int IO, int D, bool PAGED>
 void launch_mt(const LiScoreArgs& a, hipStream_t s, int MT, dim3 grid, dim3 block) {
   switch (MT) {
@@ -424,13 +635,36 @@ void launch_mt(const LiScoreArgs& a, hipStream_t s, int MT, dim3 grid, dim3 bloc
 template <int IO, int D>
 hipError_t launch_d(const LiScoreArgs& a0, hipStream_t s, int MT) {
   LiScoreArgs a = a0;
-  // Short query batches leave most CUs idle (one 8-row work-group per CU): split each row
-  // block's keys over enough work-groups for ~2 per CU, keeping at least 4 tiles each.
+  if (D == 128 && MT <= 2 && a.max_rows_per_batch <= ROWS_MAX) {
+    if (a.block_table) launch_rows<IO, true>(a, s, MT);
+    else launch_rows<IO, false>(a, s, MT);
+    return hipGetLastError();
+  }
+  // Short query batches leave CUs idle: split each row block's keys over ks work-groups. The
+  // registers hold one work-group a CU, and each costs about OVER tiles besides its own (Q, the
+  // first tiles' latency), so ks is the one with the shortest makespan: rounds of 256 equal
+  // work-groups where all rows see about the same keys, and under a causal triangle (rows up to
+  // half as many as keys and more) or over paged sequences of uneven lengths the mean work or the
+  // longest block, whichever is larger.
+  // B=1, 512 rows of 4096 keys: ks = 8 (two rounds) 41.5 us, 4 (one) 33.0; 64 rows of 16000: 16
+  // 27.3, 32 19.8; 4 x 300 rows of 5000: 4 105, 3 92; 2048 rows of 2048: 1 50, 2 40, 3 48.
+  constexpr int64_t OVER = 10;
   const int64_t blocks = (int64_t)((a.max_rows_per_batch + NW - 1) / NW) * a.n2 * a.batch;
-  const int max_tiles = (a.max_kv + LiTile<D>::BN - 1) / LiTile<D>::BN;
-  int ks = (int)((512 + blocks - 1) / blocks);
-  ks = ks < max_tiles / 4 ? ks : max_tiles / 4;
-  a.key_split = ks > 1 ? (ks < 16 ? ks : 16) : 1;
+  const int64_t tiles = (a.max_kv + LiTile<D>::BN - 1) / LiTile<D>::BN;
+  const bool causal = a.sparse_mode == 3 && 2 * (int64_t)a.max_rows_per_batch > a.max_kv;
+  const int64_t mean = causal ? tiles - (a.max_rows_per_batch / 2) / LiTile<D>::BN
+                      : a.block_table ? (tiles * 5 + 7) / 8 : tiles;
+  int64_t best = INT64_MAX;
+  a.key_split = 1;
+  for (int ks = 1; ks <= 64 && ks <= tiles; ++ks) {
+    const int64_t longest = (tiles + ks - 1) / ks + OVER;
+    const int64_t sum = blocks * (mean + OVER * ks) / 256;
+    const int64_t t = causal || a.block_table ? (sum > longest ? sum : longest) : (blocks * ks + 255) / 256 * longest;
+    if (t < best) {
+      best = t;
+      a.key_split = ks;
+    }
+  }
   dim3 grid((unsigned)(((a.max_rows_per_batch + NW - 1) / NW) * a.key_split), a.n2, a.batch), block(NW * 64);
   if (a.block_table)
     launch_mt<IO, D, true>(a, s, MT, grid, block);

@@ -436,3 +436,35 @@ def test_topk_order_of_nan_and_signed_zero_patterns(dev, S1, S2, K):
         ev = np.where(bits[r, order] == 0x8000, 0, bits[r, order])
         assert np.array_equal(gv[r, :n], ev), (S2, r, L)
         assert np.all(gv[r, n:] == 0)
+
+
+@pytest.mark.parametrize("S1,N1,N2", [(1, 64, 1), (2, 8, 1), (3, 80, 2), (4, 33, 1), (5, 64, 1)])
+@pytest.mark.parametrize("page", [None, 16, 48, 64])
+def test_few_query_rows(dev, S1, N1, N2, page):
+    """One to four query rows a batch (decode; five take the general kernel): key counts at the
+    edges of the 32-key subtile and of the work-group's chunk, several key heads, partial head
+    tiles, pages smaller and larger than a subtile with a missing one, each score against the
+    oracle."""
+    rng = np.random.RandomState(21)
+    D, K, dtype = 128, 4400, "fp16"
+    lens = [S1, 31, 32, 33, 255, 257, 1023, 2049, 4100]
+    B = len(lens)
+    q = torch.from_numpy(rng.randn(B, S1, N1, D).astype(np.float32)).to(DT[dtype])
+    w = torch.from_numpy(rng.randn(B, S1, N1).astype(np.float32))
+    if page is None:
+        dense = torch.from_numpy(rng.randn(B, max(lens), N2, D).astype(np.float32)).to(DT[dtype])
+        idx, val = lightning_indexer(q.to(dev), dense.to(dev), w.to(dev), actual_seq_lengths_key=lens,
+                                     sparse_count=K, sparse_mode=3, return_value=True)
+        dense = _np(dense)
+    else:
+        bt, cache, dense = _paged(rng, B, lens, page, N2, D, dtype, missing=(6, 3))
+        idx, val = lightning_indexer(q.to(dev), cache.to(dev), w.to(dev), actual_seq_lengths_key=lens,
+                                     block_table=bt.to(dev), layout_key="PA_BSND", sparse_count=K, sparse_mode=3,
+                                     return_value=True)
+    torch.cuda.synchronize()
+    gi, gv = idx.cpu().numpy(), val.float().cpu().numpy()
+    S2, ak = dense.shape[1], np.asarray(lens)
+    Ls = np.concatenate([np.repeat(_visible(S1, S2, S1, ak[b], 3), N2) for b in range(B)])
+    check_topk_properties(gi.reshape(-1, K), gv.reshape(-1, K), Ls, K)
+    stats = check_li(gi, gv, _np(q), dense, _np(w), np.full(B, S1), ak, K, 3, dtype)
+    assert stats.flips <= max(4, 0.02 * stats.elements), stats
