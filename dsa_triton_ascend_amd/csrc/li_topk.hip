@@ -33,14 +33,14 @@
 //   5. One pass writes the indices and 16-bit values in rank order.
 // The selection histogram and the sort's counters share one LDS array (they are
 // never live together), so a work-group needs ~16 KB and more of them fit a CU.
+#include <type_traits>
+
 #include "dsa_common.hpp"
 
 namespace dsa {
 namespace {
 
-constexpr int TPB = 256;
-constexpr int RPT = 32;                 // row entries per thread held in VGPRs
-constexpr int ROW_CACHED = TPB * RPT;   // 8192
+constexpr int ROW_CACHED = 8192;   // row entries that 256 threads hold in VGPRs, 32 each
 
 __device__ __forceinline__ int visible_len(int s1, int aq, int ak, int S2, int mode) {
   int L;
@@ -60,6 +60,7 @@ __device__ __forceinline__ int visible_len(int s1, int aq, int ak, int S2, int m
 // last scan's) and this call (the compaction and candidate scans follow the barriers of
 // the bin pick and of the candidate resolution, each sort pass's scan the pass's count
 // barrier), so the words are free to overwrite.
+template <int TPB>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* red, uint32_t* total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t x = wave_incl_sum(v);
@@ -118,8 +119,9 @@ __device__ __forceinline__ void lds_push(lds_u32*& p, uint32_t v) {
 // key e of a thread's packed pairs (w[e / 2], low half = even e)
 __device__ __forceinline__ uint32_t kh(const uint32_t* w, int e) { return (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xFFFFu; }
 
-// Keys [base + 32t, +32) of the row as packed ord16 pairs; entries at or past L are 0
+// Keys [base + RPT t, +RPT) of the row as packed ord16 pairs; entries at or past L are 0
 // (below every real key). Threads whose entries all lie past L load nothing.
+template <int RPT>
 __device__ __forceinline__ void load_keys(const uint16_t* row, int L, int base, uint32_t (&w)[RPT / 2]) {
   const int i0 = base + threadIdx.x * RPT;
   if (i0 + RPT <= L) {
@@ -160,7 +162,7 @@ __device__ __forceinline__ int rank_block(int t) { return (t & ~63) | ((t & 31) 
 // never read back): they stay behind every real key in each pass, so they affect no
 // real key's position, and a wave holding padding only neither counts nor moves it
 // (the ranks past the active waves' slots are then left stale).
-template <int E>
+template <int TPB, int E>
 __device__ __forceinline__ void radix_sort_asc16(uint32_t (&key)[E], int npass, int n, uint32_t* sbuf,
                                                  uint16_t* cnt, uint32_t* red) {
   const int t = threadIdx.x, tb = rank_block(t);
@@ -192,7 +194,7 @@ __device__ __forceinline__ void radix_sort_asc16(uint32_t (&key)[E], int npass, 
     for (int j = 0; j < 8; ++j) s += w[j];
     s = (s & 0xFFFFu) + (s >> 16);
     uint32_t tot;
-    uint32_t run = block_excl_scan(s, red, &tot);   // offset of this thread's first entry
+    uint32_t run = block_excl_scan<TPB>(s, red, &tot);   // offset of this thread's first entry
     uint32_t o[8];   // running offsets, re-derived from the counts (no second array live across the scan)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -225,7 +227,7 @@ __device__ __forceinline__ void radix_sort_asc16(uint32_t (&key)[E], int npass, 
 // gets the scan total and both maxima): one LDS exchange for the three. LEAD: a barrier
 // first, for callers whose threads may still be reading `red` from an earlier scan (a
 // caller's first scan of the row needs none). M2 = false: m2 is unused (max2 gets 0).
-template <bool LEAD = true, bool M2 = true>
+template <int TPB, bool LEAD = true, bool M2 = true>
 __device__ __forceinline__ uint32_t block_scan_max2(uint32_t v, uint32_t m1, uint32_t m2, uint32_t* red,
                                                     uint32_t* total, uint32_t* max1, uint32_t* max2) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -259,11 +261,12 @@ __device__ __forceinline__ uint32_t block_scan_max2(uint32_t v, uint32_t m1, uin
 // which cost less than the latency an eighth work-group per CU hides). At eight waves per
 // SIMD the VALU issues for about two thirds of the kernel's time; LDS bank conflicts and
 // the chain of block barriers take most of the rest.
-template <int E, bool WIDE, bool SHORT = false>
-__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(SHORT && E <= 8 ? 8 : 1, 8)))
+template <int TPB, int RPT, int E, bool WIDE, bool SHORT>
+__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(TPB == 256 ? (SHORT && E <= 8 ? 8 : 1) : 4, 8)))
 void li_topk_kernel(LiTopkArgs a) {
   static_assert(!(SHORT && WIDE), "short rows use 16-bit indices");
-  static_assert(E * TPB <= 65536, "compacted positions are 16-bit");
+  static_assert(E * TPB <= 65536 && TPB * RPT <= 32768, "compacted positions and packed counts are 16-bit");
+  constexpr int ROW_CACHED = TPB * RPT;   // row entries held in VGPRs
   constexpr int HWORDS = 2048;         // selection histogram (u >> 5), then the candidate list
   constexpr int CWORDS = 16 * TPB / 2;   // sort counters (16-bit)
   __shared__ __attribute__((aligned(16))) uint32_t sbuf[E * TPB];
@@ -299,7 +302,7 @@ void li_topk_kernel(LiTopkArgs a) {
   // ---- selection + order-preserving compaction into sbuf[0, nout)
   const int nchunks = SHORT ? 1 : (L + ROW_CACHED - 1) / ROW_CACHED;
   uint32_t w[RPT / 2];   // the thread's keys, packed pairs
-  if (nchunks == 1) load_keys(row, L, 0, w);
+  if (nchunks == 1) load_keys<RPT>(row, L, 0, w);
   // one chunk: whether this wave holds any entry of the row (the per-entry loops of the
   // others are skipped: every key they hold is 0)
   const bool wv = nchunks > 1 || __builtin_amdgcn_readfirstlane(t >> 6) * 64 * RPT < L;
@@ -310,12 +313,14 @@ void li_topk_kernel(LiTopkArgs a) {
   if (L > k) {
     // 2048-bin histogram of u >> 5, scanned from the top bin: bin b holds the k-th
     // largest key, `above` keys lie in higher bins (all taken)
+    constexpr int HB = HWORDS / TPB;   // bins per thread: 8 or 2
+    static_assert(HB == 8 || HB == 2, "");
 #pragma unroll
-    for (int i = 0; i < 8; ++i) hist[t * 8 + i] = 0;
+    for (int i = 0; i < HB; ++i) hist[t * HB + i] = 0;
     __syncthreads();
 #pragma unroll 1
     for (int ch = 0; ch < nchunks; ++ch) {
-      if (nchunks > 1) load_keys(row, L, ch * ROW_CACHED, w);
+      if (nchunks > 1) load_keys<RPT>(row, L, ch * ROW_CACHED, w);
       // every key of a thread holding part of the row is counted, with no per-key test:
       // the padding past L of the one thread straddling L lands in bin 0 and is taken
       // out below (threads wholly past L count nothing, so bin 0 sees no pile-up)
@@ -328,26 +333,29 @@ void li_topk_kernel(LiTopkArgs a) {
         }
     }
     __syncthreads();
-    uint32_t h[8];   // thread t: bins 2047 - 8t - j, j < 8 (the scan runs from the top)
-    {
+    uint32_t h[HB];   // thread t: bins 2047 - HB t - j, j < HB (the scan runs from the top)
+    if constexpr (HB == 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(&hist[2046 - 2 * t]);
+      h[0] = v.y; h[1] = v.x;
+    } else {
       const uint4 lo4 = *reinterpret_cast<const uint4*>(&hist[2040 - 8 * t]);
       const uint4 hi4 = *reinterpret_cast<const uint4*>(&hist[2044 - 8 * t]);
       h[0] = hi4.w; h[1] = hi4.z; h[2] = hi4.y; h[3] = hi4.x;
       h[4] = lo4.w; h[5] = lo4.z; h[6] = lo4.y; h[7] = lo4.x;
     }
-    if (t == TPB - 1) h[7] -= (uint32_t)(-L & (RPT - 1));   // bin 0: the padding counted above
+    if (t == TPB - 1) h[HB - 1] -= (uint32_t)(-L & (RPT - 1));   // bin 0: the padding counted above
     uint32_t hs = 0, top1 = 0;   // top1: highest non-empty bin + 1 (0: none)
 #pragma unroll
-    for (int j = 7; j >= 0; --j) {
+    for (int j = HB - 1; j >= 0; --j) {
       hs += h[j];
-      top1 = h[j] ? (uint32_t)(2048 - 8 * t - j) : top1;
+      top1 = h[j] ? (uint32_t)(2048 - HB * t - j) : top1;
     }
     uint32_t tot, btop1, unused;
-    uint32_t cum = block_scan_max2<false, false>(hs, top1, 0u, red, &tot, &btop1, &unused);
+    uint32_t cum = block_scan_max2<TPB, false, false>(hs, top1, 0u, red, &tot, &btop1, &unused);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < HB; ++j) {
       if (cum < (uint32_t)k && cum + h[j] >= (uint32_t)k) {
-        pick[0] = 2047 - 8 * t - j;
+        pick[0] = 2047 - HB * t - j;
         pick[1] = cum;
         pick[2] = h[j];
       }
@@ -396,7 +404,7 @@ void li_topk_kernel(LiTopkArgs a) {
         }
       const uint32_t cg = pk_hsum(ag), cc = pk_hsum(ab) - cg;
       uint32_t tot1;
-      const uint32_t pgc = block_excl_scan((cg << 16) | cc, red, &tot1);
+      const uint32_t pgc = block_excl_scan<TPB>((cg << 16) | cc, red, &tot1);
       lds_u32* ps = (lds_u32*)(sbuf + (pgc >> 16));
       lds_u32* pcd = (lds_u32*)(cand + (pgc & 0xFFFFu));
       const uint32_t xb = 0xFFFFu - (uint32_t)i0;
@@ -414,30 +422,31 @@ void li_topk_kernel(LiTopkArgs a) {
           if (hi) lds_push(ps, v);               // a higher bin
           if (ue > b1 && !hi) lds_push(pcd, v);  // bin `bin`, nonzero
         }
-      // candidates [c0, c1) of this thread (at most 8: nc <= 2048; the loops stop at the
+      // candidates [c0, c1) of this thread (at most MC: nc <= 2048; the loops stop at the
       // block-uniform m, typically 1 or 2)
+      constexpr int MC = HWORDS / TPB;
       const uint32_t m = (nc + TPB - 1) / TPB, c0 = min((uint32_t)t * m, nc), c1 = min(c0 + m, nc);
       resolve([&] {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < MC; ++j) {
           if (j >= (int)m) break;
           if (c0 + j < c1) atomicAdd(&chist[(cand[c0 + j] >> 16) & 31u], 1u);
         }
       });
-      uint32_t cv[8];
+      uint32_t cv[MC];
       uint32_t g2 = 0, e2 = 0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < MC; ++j) {
         if (j >= (int)m) break;
         cv[j] = c0 + j < c1 ? cand[c0 + j] : 0u;
         g2 += (c0 + j < c1 && (cv[j] >> 16) > T) ? 1u : 0u;
         e2 += (c0 + j < c1 && (cv[j] >> 16) == T) ? 1u : 0u;
       }
       uint32_t tot2;
-      const uint32_t pge = block_excl_scan((g2 << 16) | e2, red, &tot2);
+      const uint32_t pge = block_excl_scan<TPB>((g2 << 16) | e2, red, &tot2);
       uint32_t qg = above + (pge >> 16), qe = pge & 0xFFFFu;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < MC; ++j) {
         if (j >= (int)m) break;
         if (c0 + j >= c1) continue;
         const uint32_t key16 = cv[j] >> 16, x = cv[j] & 0xFFFFu;
@@ -454,7 +463,7 @@ void li_topk_kernel(LiTopkArgs a) {
       resolve([&] {
 #pragma unroll 1
         for (int ch = 0; ch < nchunks; ++ch) {
-          if (nchunks > 1) load_keys(row, L, ch * ROW_CACHED, w);
+          if (nchunks > 1) load_keys<RPT>(row, L, ch * ROW_CACHED, w);
 #pragma unroll
           for (int e = 0; e < RPT; ++e)
             if (kh(w, e) != 0u && (kh(w, e) >> 5) == bin) atomicAdd(&chist[kh(w, e) & 31u], 1u);
@@ -492,7 +501,7 @@ void li_topk_kernel(LiTopkArgs a) {
           if (i0 + e < L) sbuf[i0 + e] = (kh(w, e) << 16) | (0xFFFFu - (uint32_t)(i0 + e));
       }
       uint32_t tot, cmx, cmn;
-      block_scan_max2<false>(0u, mx, mninv, red, &tot, &cmx, &cmn);
+      block_scan_max2<TPB, false>(0u, mx, mninv, red, &tot, &cmx, &cmn);
       umax = cmx;
       umin = 0xFFFFu - cmn;
       compacted = true;
@@ -506,7 +515,7 @@ void li_topk_kernel(LiTopkArgs a) {
     uint32_t kmax = 0, kmin_inv = 0;   // max of u, max of 0xFFFF - u over nonzero keys
 #pragma unroll 1
     for (int ch = 0; ch < nchunks; ++ch) {
-      if (nchunks > 1) load_keys(row, L, ch * ROW_CACHED, w);
+      if (nchunks > 1) load_keys<RPT>(row, L, ch * ROW_CACHED, w);
       const int i0 = ch * ROW_CACHED + t * RPT;
       uint32_t cg = 0, ce = 0, mx = 0, mn = 0;
 #pragma unroll
@@ -518,7 +527,7 @@ void li_topk_kernel(LiTopkArgs a) {
         mn = ue != 0u ? max(mn, 0xFFFFu - ue) : mn;
       }
       uint32_t tot, cmx, cmn;
-      const uint32_t pgs = block_scan_max2((cg << 16) | ce, mx, mn, red, &tot, &cmx, &cmn);
+      const uint32_t pgs = block_scan_max2<TPB>((cg << 16) | ce, mx, mn, red, &tot, &cmx, &cmn);
       kmax = max(kmax, cmx);
       kmin_inv = max(kmin_inv, cmn);
       uint32_t pg = (pgs >> 16) + run_g;
@@ -568,7 +577,7 @@ void li_topk_kernel(LiTopkArgs a) {
     const uint32_t x = sbuf[E * tb + e];
     key[e] = (min(umax - (x >> 16), vmax) << 16) | (x & 0xFFFFu);
   }
-  radix_sort_asc16<E>(key, npass, nout, sbuf, cnt, red);
+  radix_sort_asc16<TPB, E>(key, npass, nout, sbuf, cnt, red);
   // ranks E tb .. E tb + E - 1 of thread t: their index (or -1) and 16-bit value (or 0).
   // A run of 8 ranks inside the row's output, all below nout (the usual case): indices
   // 0xFFFF - x, values unord16(umax - v) computed on packed pairs.
@@ -606,18 +615,27 @@ void li_topk_kernel(LiTopkArgs a) {
     else oi[e] = ok ? (int32_t)(0xFFFFu - (key[e] & 0xFFFFu)) : -1;
     ov[e] = ok ? unord16(umax - (key[e] >> 16)) : (uint16_t)0;
   }
-  // 16-byte stores when the thread's whole run lies inside the row and rows are
-  // 16-byte aligned (k % 8 == 0); the rest element by element
-  if (E % 8 == 0 && k % 8 == 0 && E * tb + E <= k) {
+  // wide stores when the thread's whole run lies inside the row and rows are aligned to
+  // them (up to four indices, eight values); the rest element by element
+  constexpr int VI = E % 4 == 0 ? 4 : (E % 2 == 0 ? 2 : 1), VV = E % 8 == 0 ? 8 : VI;
+  if (E > 1 && k % VV == 0 && E * tb + E <= k) {
+    int32_t* io = iout + E * tb;
 #pragma unroll
-    for (int e = 0; e < E; e += 4)
-      *reinterpret_cast<int4*>(iout + E * tb + e) = make_int4(oi[e], oi[e + 1], oi[e + 2], oi[e + 3]);
-    if (vout)
+    for (int e = 0; e < E; e += VI) {
+      if constexpr (VI == 4) *reinterpret_cast<int4*>(io + e) = make_int4(oi[e], oi[e + 1], oi[e + 2], oi[e + 3]);
+      else if constexpr (VI == 2) *reinterpret_cast<int2*>(io + e) = make_int2(oi[e], oi[e + 1]);
+    }
+    if (vout) {
+      uint16_t* vo = vout + E * tb;
+      auto two = [&](int e) { return ov[e] | ((uint32_t)ov[e + 1] << 16); };
 #pragma unroll
-      for (int e = 0; e < E; e += 8)
-        *reinterpret_cast<uint4*>(vout + E * tb + e) =
-            make_uint4(ov[e] | ((uint32_t)ov[e + 1] << 16), ov[e + 2] | ((uint32_t)ov[e + 3] << 16),
-                       ov[e + 4] | ((uint32_t)ov[e + 5] << 16), ov[e + 6] | ((uint32_t)ov[e + 7] << 16));
+      for (int e = 0; e < E; e += VV) {
+        if constexpr (VV == 8)
+          *reinterpret_cast<uint4*>(vo + e) = make_uint4(two(e), two(e + 2), two(e + 4), two(e + 6));
+        else if constexpr (VV == 4) *reinterpret_cast<uint2*>(vo + e) = make_uint2(two(e), two(e + 2));
+        else if constexpr (VV == 2) *reinterpret_cast<uint32_t*>(vo + e) = two(e);
+      }
+    }
   } else {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -753,16 +771,24 @@ __global__ __launch_bounds__(BIG_TPB) void li_topk_big_kernel(LiTopkArgs a, uint
 }  // namespace
 }  // namespace dsa
 
-template <bool WIDE, bool SHORT>
-static hipError_t launch_topk_e(const LiTopkArgs& a, int e, unsigned rows, hipStream_t s) {
-  const dim3 grid(rows), block(dsa::TPB);
-  if (e <= 1) hipLaunchKernelGGL((dsa::li_topk_kernel<1, WIDE, SHORT>), grid, block, 0, s, a);
-  else if (e <= 2) hipLaunchKernelGGL((dsa::li_topk_kernel<2, WIDE, SHORT>), grid, block, 0, s, a);
-  else if (e <= 4) hipLaunchKernelGGL((dsa::li_topk_kernel<4, WIDE, SHORT>), grid, block, 0, s, a);
-  else if (e <= 8) hipLaunchKernelGGL((dsa::li_topk_kernel<8, WIDE, SHORT>), grid, block, 0, s, a);
-  else if (e <= 16) hipLaunchKernelGGL((dsa::li_topk_kernel<16, WIDE, SHORT>), grid, block, 0, s, a);
-  else if (e <= 32) hipLaunchKernelGGL((dsa::li_topk_kernel<32, WIDE, SHORT>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((dsa::li_topk_kernel<64, WIDE, SHORT>), grid, block, 0, s, a);
+template <int TPB, int RPT, bool WIDE, bool SHORT, int EMAX>
+static hipError_t launch_topk_e(const LiTopkArgs& a, unsigned rows, hipStream_t s) {
+  const int e = (a.k + TPB - 1) / TPB;
+  const dim3 grid(rows), block(TPB);
+  auto go = [&](auto ec) {
+    hipLaunchKernelGGL((dsa::li_topk_kernel<TPB, RPT, decltype(ec)::value, WIDE, SHORT>), grid, block, 0, s, a);
+  };
+  if (e <= 1) go(std::integral_constant<int, 1>{});
+  else if (e <= 2) go(std::integral_constant<int, 2>{});
+  else if (e <= 4) go(std::integral_constant<int, 4>{});
+  else if constexpr (EMAX >= 8) {
+    if (e <= 8) go(std::integral_constant<int, 8>{});
+    else if constexpr (EMAX >= 64) {
+      if (e <= 16) go(std::integral_constant<int, 16>{});
+      else if (e <= 32) go(std::integral_constant<int, 32>{});
+      else go(std::integral_constant<int, 64>{});
+    }
+  }
   return hipGetLastError();
 }
 
@@ -782,8 +808,26 @@ hipError_t launch_li_topk_big(const LiTopkArgs& a, void* ws, hipStream_t s) {
 hipError_t launch_li_topk(const LiTopkArgs& a, hipStream_t s) {
   const int64_t rows = (int64_t)a.total_rows * a.n2;
   if (rows <= 0) return hipSuccess;
-  const int e = (a.k + dsa::TPB - 1) / dsa::TPB;
-  if (a.s2 > 65536) return launch_topk_e<true, false>(a, e, (unsigned)rows, s);
-  if (a.s2 > dsa::ROW_CACHED) return launch_topk_e<false, false>(a, e, (unsigned)rows, s);
-  return launch_topk_e<false, true>(a, e, (unsigned)rows, s);   // every visible row fits the registers
+  const unsigned n = (unsigned)rows;
+  // Few rows (a decode step) leave most of the chip idle and the call's time is one row's latency:
+  // 1024 threads a row, which hold up to 32768 entries in registers (one pass over the row instead
+  // of three in chunks of 8192). 64 rows of 4K .. 32K entries: 31.8 -> 16.5 us; 256 rows of 5000:
+  // 13.1 -> 11.8, of 20000: 32.2 -> 17.6, of 40000: 45 -> 33. With a second work-group a CU the
+  // shorter throughput of 256 threads wins for rows that fit its registers (400 rows of 5000: 15.1
+  // against 16.7) and for rows of several chunks (40000: 55 against 60), not between (512 rows of
+  // 20000: 41.5 against 31.1).
+  if (rows <= 512 && a.k <= 4096) {
+    if (a.s2 > dsa::ROW_CACHED && a.s2 <= 32768) return launch_topk_e<1024, 32, false, true, 4>(a, n, s);
+    if (rows <= 256) {
+      if (a.s2 > 65536) return launch_topk_e<1024, 32, true, false, 4>(a, n, s);
+      if (a.s2 > 32768) return launch_topk_e<1024, 32, false, false, 4>(a, n, s);
+      if (a.s2 > 2048) return launch_topk_e<1024, 8, false, true, 4>(a, n, s);
+    }
+  }
+  // Short rows: eight entries a thread spread the per-entry loops over four times the threads
+  // (256 rows of 256 entries: 10.7 -> 7.4 us; 1024 rows of 1500: 15.4 -> 12.2)
+  if (a.s2 <= 2048 && a.k <= 2048) return launch_topk_e<256, 8, false, true, 8>(a, n, s);
+  if (a.s2 > 65536) return launch_topk_e<256, 32, true, false, 64>(a, n, s);
+  if (a.s2 > dsa::ROW_CACHED) return launch_topk_e<256, 32, false, false, 64>(a, n, s);
+  return launch_topk_e<256, 32, false, true, 64>(a, n, s);   // every visible row fits the registers
 }

@@ -438,6 +438,18 @@ def test_topk_order_of_nan_and_signed_zero_patterns(dev, S1, S2, K):
         assert np.all(gv[r, n:] == 0)
 
 
+@pytest.mark.parametrize("S1,S2,K", [(520, 12000, 2048), (300, 40000, 2048), (257, 70000, 1024),   # 256 threads, chunked
+                                     (20, 2049, 2048), (256, 8192, 1000), (9, 5000, 4096),         # 1024 threads, 8 each
+                                     (512, 8193, 2048), (7, 32768, 513),                           # 1024 threads, 32 each
+                                     (6, 32769, 2048), (5, 65537, 4096),                           # ... in chunks
+                                     (700, 2048, 2048), (40, 257, 300), (33, 7, 5)])               # 256 threads, 8 each
+@pytest.mark.parametrize("family", ["two_values", "wide"])
+def test_topk_instances_by_rows_and_length(dev, S1, S2, K, family):
+    """Every instance of the top-k's dispatch (threads a row and entries a thread, by rows,
+    S2 and k) at the edges of its range, bit for bit against the golden's stable sort."""
+    test_topk_crafted_score_rows(dev, S1, S2, K, family)
+
+
 @pytest.mark.parametrize("S1,N1,N2", [(1, 64, 1), (2, 8, 1), (3, 80, 2), (4, 33, 1), (5, 64, 1)])
 @pytest.mark.parametrize("page", [None, 16, 48, 64])
 def test_few_query_rows(dev, S1, N1, N2, page):
