@@ -143,6 +143,34 @@ __device__ __forceinline__ f32x16 mfma32_vacc_last_to(const f32x16& c, uint4 a, 
   return d;
 }
 
+// Two 16x16x32 chains that share their A operand (accumulators c0, c1 in arch VGPRs, B operands b0,
+// b1), one step of both per statement; rules as for the 32x32 chains above. DRAIN: the last step.
+#define DSA_MFMA16_PAIR(T, C0, C1, TAIL) \
+  "v_mfma_f32_16x16x32_" T " %0, %2, %3, " C0 "\n\tv_mfma_f32_16x16x32_" T " %1, %2, %4, " C1 TAIL
+template <int IO>
+__device__ __forceinline__ void mfma16x2_vacc_first(f32x4& c0, f32x4& c1, uint4 a, uint4 b0, uint4 b1) {
+  const i32x4v av = __builtin_bit_cast(i32x4v, a), bv0 = __builtin_bit_cast(i32x4v, b0),
+               bv1 = __builtin_bit_cast(i32x4v, b1);
+  if constexpr (IO == IO_BF16)
+    asm volatile(DSA_MFMA16_PAIR("bf16", "0", "0", "") : "=&v"(c0), "=&v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+  else
+    asm volatile(DSA_MFMA16_PAIR("f16", "0", "0", "") : "=&v"(c0), "=&v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+}
+template <int IO, bool DRAIN>
+__device__ __forceinline__ void mfma16x2_vacc(f32x4& c0, f32x4& c1, uint4 a, uint4 b0, uint4 b1) {
+  const i32x4v av = __builtin_bit_cast(i32x4v, a), bv0 = __builtin_bit_cast(i32x4v, b0),
+               bv1 = __builtin_bit_cast(i32x4v, b1);
+  if constexpr (IO == IO_BF16 && DRAIN)
+    asm volatile(DSA_MFMA16_PAIR("bf16", "%0", "%1", "\n\ts_nop 15\n\ts_nop 1") : "+v"(c0), "+v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+  else if constexpr (IO == IO_BF16)
+    asm volatile(DSA_MFMA16_PAIR("bf16", "%0", "%1", "") : "+v"(c0), "+v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+  else if constexpr (DRAIN)
+    asm volatile(DSA_MFMA16_PAIR("f16", "%0", "%1", "\n\ts_nop 15\n\ts_nop 1") : "+v"(c0), "+v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+  else
+    asm volatile(DSA_MFMA16_PAIR("f16", "%0", "%1", "") : "+v"(c0), "+v"(c1) : "v"(av), "v"(bv0), "v"(bv1));
+}
+#undef DSA_MFMA16_PAIR
+
 // Output layouts (CDNA3/CDNA4 MFMA, 64 lanes):
 //  32x32: lane l, acc[r] (r < 16) holds C[row = (r/4)*8 + (l/32)*4 + r%4][col = l%32]
 //  16x16: lane l, acc[r] (r < 4)  holds C[row = (l/16)*4 + r][col = l%16]
@@ -224,6 +252,12 @@ __device__ __forceinline__ float max_half_swap(float x) {
 // s_nop 1 gives the wait states the swap needs after VALU writes of its operands.
 __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+
+// v_permlane16_swap: exchanges the odd 16-lane rows of `a` with the even rows of `b`: afterwards
+// a[16 + l] = old b[l], b[l] = old a[16 + l] (l < 16), and the same between lanes 32 .. 63.
+__device__ __forceinline__ void swap_rows16(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
 
 // Wave-wide inclusive prefix sum / max over the 64 lanes with DPP, VALU only (the

@@ -1467,9 +1467,409 @@ __global__ __launch_bounds__(NWV * 64) void sfa_attn_kernel(SfaArgs a, int cap, 
   }
 }
 
+// ---------------------------------------------------------------- kernel 2, per-wave form of up to 64 heads (D = 512)
+// The per-wave PV form above on two waves: a work-group per (query row, KV split), every wave running
+// S^T, the softmax and PV of its own 32 heads over all columns, P in its registers. Two work-groups
+// share a CU (one wave per SIMD each: O^T takes 256 AGPRs, Q^T with its rope 144 VGPRs), so a CU
+// works on two query rows at once and one row's prologue and epilogue run beside the other's tiles.
+// A pair of tiles takes about 4,650 cycles against 2,176 of MFMA, the same as the 128-head form (and
+// without its gathers, 15%, the chip's clock under this load is most of what is left); the eight-wave
+// form this replaces took 3,600 per single tile.
+//  * The ring holds two 32-token tiles (two work-groups' rings fill the LDS): the gathers of tile t+1
+//    ride on the S^T chain of tile t and have its softmax and PV to land. One barrier per tile.
+//  * Rows are unpadded (1024 B) and 16-byte chunk c of token t sits at c ^ swz(t), a bijection of
+//    t % 16 chosen for both readers: the 8 consecutive tokens of an S^T operand read differ in its low
+//    three bits, and the four tokens of a transposed V read in bits 2 and 3, so their 64-byte runs
+//    cover all 64 banks.
+//  * A tile's scores come in two halves of 16 tokens (16x16x32 MFMAs, two head tiles sharing each K
+//    operand): the softmax of the first half runs under the S^T MFMAs of the second, that of the second
+//    under the PV MFMAs of the first. The last NPRE PV MFMAs of a tile run after the next barrier, under
+//    the next tile's first LDS reads.
+namespace w2 {
+constexpr int D = 512;
+constexpr int NW = 2;                             // waves, 32 heads each
+constexpr int KS = (D + DR) / 32, KSN = D / 32;   // S^T k-steps (18), of which nope (16)
+constexpr int NOPE = BN * D * 2;                  // bytes of a tile's nope rows
+constexpr int ROPE = BN * DR * 2;
+__host__ __device__ constexpr int swz(int t) {
+  return ((((t >> 1) ^ (t >> 3)) & 1) << 3) | ((t & 1) << 2) | (t & 2) | ((t >> 2) & 1);
+}
+}  // namespace w2
+
+// f(integral_constant I), f(I + 1), .. f(N - 1): an unrolled loop whose body may be of any size (the
+// compiler gives up on `#pragma unroll` of very large ones and moves the arrays they index to scratch)
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+template <int IO>
+__global__ __launch_bounds__(w2::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
+  using w2::D;
+  using w2::NW;
+  constexpr int KS = w2::KS, KSN = w2::KSN;
+  constexpr int RPW = BN / NW;          // token rows a wave gathers per tile
+  constexpr int RG = RPW / 8;           // rope loads (8 tokens each)
+  constexpr int GPW = RPW + RG + 1;     // loads per wave per tile: nope rows, rope, ids
+  __shared__ __attribute__((aligned(1024))) uint8_t nope_buf[2][w2::NOPE];   // before the first gathers: Q^T nope
+  __shared__ __attribute__((aligned(16))) uint8_t rope_buf[2][w2::ROPE];
+  __shared__ __attribute__((aligned(16))) int32_t s_ids[4][BN];   // token-id ring (tiles t+2 .. t+4)
+  static_assert(NW * 32 * D * 2 <= 2 * w2::NOPE, "Q^T staging");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = a.total_rows - 1 - (int)blockIdx.x;   // long (late causal) rows first
+  const int sp = blockIdx.y;
+  const int n1 = a.n1;
+  const float cpos = a.scale > 0.f ? a.scale : a.scale < 0.f ? -a.scale : 1e-30f;
+  const float cl2 = cpos * LOG2E;
+  const int ntok_all = ws.counts[r];
+  const int hq = wave * 32 + (lane & 31);
+  const int kg = lane >> 5;
+  const int32_t* toks0 = ws.tokens + (int64_t)r * ws.tstride;
+  // the ids of tiles 0..3 and Q are requested before the token count arrives (see sfa_attn_kernel)
+  const bool early_ids = splits == 1;
+  auto ids_copy = [&](const int32_t* src, int slot) {
+    if (lane < RPW / 4) lds_dma16_sbase_untracked(src + wave * RPW, lane * 16, &s_ids[slot][wave * RPW]);
+  };
+  if (early_ids)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if ((t + 1) * BN <= ws.tstride) ids_copy(toks0 + t * BN, t);
+  {
+    const uint16_t* q0 = reinterpret_cast<const uint16_t*>(a.q) + (int64_t)r * n1 * D;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {   // one head row per copy, chunk c at c ^ (head % 16)
+      const int h = min(wave * 32 + j, n1 - 1);
+      lds_dma16_sbase_untracked(q0 + (int64_t)h * D, (uint32_t)(lane ^ (j & 15)) * 16,
+                                &nope_buf[0][0] + (wave * 32 + j) * (D * 2));
+    }
+  }
+  const int l16 = lane & 15, g4 = lane >> 4;
+  // Q^T fragments: head wave * 32 + 16 n + lane % 16, 8 elements at 32 ks + 8 (lane / 16)
+  uint4 qf[KS][2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const uint16_t* qr =
+        reinterpret_cast<const uint16_t*>(a.qr) + ((int64_t)r * n1 + min(wave * 32 + 16 * n + l16, n1 - 1)) * DR;
+#pragma unroll
+    for (int j = KSN; j < KS; ++j) qf[j][n] = ldg16(qr + (j - KSN) * 32 + g4 * 8);
+  }
+  asm volatile("" ::: "memory");   // the loads stay ahead of the token-count branch
+
+  const int per = ((ntok_all + splits - 1) / splits + BN - 1) / BN * BN;
+  const int t_beg = sp * per;
+  const int t_end = (t_beg + per < ntok_all ? t_beg + per : ntok_all);
+  const int ntok = t_end > t_beg ? t_end - t_beg : 0;
+  const int32_t* toks = toks0 + t_beg;
+  uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
+  if (ntok == 0) {
+    wait_vmcnt<0>();
+    if (ntok_all == 0 && sp == 0) {   // skipped row: zeros (out, stats)
+      for (int i = threadIdx.x; i < n1 * D / 8; i += NW * 64)
+        stg16(out + (int64_t)r * n1 * D + i * 8, make_uint4(0, 0, 0, 0));
+      if (a.sm_max)
+        for (int h = threadIdx.x; h < n1; h += NW * 64) {
+          a.sm_max[(int64_t)r * n1 + h] = 0.f;
+          a.sm_sum[(int64_t)r * n1 + h] = 0.f;
+        }
+    }
+    return;
+  }
+  const int nact = (ntok_all + per - 1) / per;
+  const bool direct = nact == 1;
+  const uint16_t* kb = reinterpret_cast<const uint16_t*>(a.k);
+  const uint16_t* krb = reinterpret_cast<const uint16_t*>(a.kr);
+  const int krows = a.key_rows < INT_MAX ? (int)a.key_rows : INT_MAX;
+  const int ntiles = (ntok + BN - 1) / BN;
+  auto clamp_tile = [&](int t) { return t < ntiles ? t : ntiles - 1; };
+  auto ids_dma = [&](int t) { ids_copy(toks + clamp_tile(t) * BN, t & 3); };
+  struct Idx {
+    int nope;       // lane: token lane % RPW of the wave
+    int rope[RG];   // lane: token 8 j + lane % 8
+    uint32_t zero_rows;   // nope rows whose id is out of range: they read row 0 and are zeroed once landed
+  };
+  auto tile_idx = [&](int t) __attribute__((always_inline)) {
+    const int tb = clamp_tile(t) * BN;
+    const int nvalid = ntok - tb < BN ? ntok - tb : BN;
+    const int32_t* ids = s_ids[t & 3];
+    const int first = ids[0];   // slots past the token list take the tile's first token
+    const int k = wave * RPW + (lane & (RPW - 1));
+    int v = ids[k];
+    Idx ix;
+#pragma unroll
+    for (int j = 0; j < RG; ++j) {
+      const int k2 = wave * RPW + 8 * j + (lane & 7);
+      const int u = ids[k2];
+      ix.rope[j] = k2 < nvalid ? u : first;   // the rope gather selects the zero row itself
+    }
+    v = k < nvalid ? v : first;
+    const bool bad = (uint32_t)v >= (uint32_t)krows;
+    ix.zero_rows = (uint32_t)__builtin_amdgcn_ballot_w64(bad) & (uint32_t)((1ull << RPW) - 1);
+    ix.nope = bad ? 0 : v;
+    return ix;
+  };
+  // gather part j of a tile: j < RPW the nope row of the wave's token j, then RG rope groups
+  auto gather_part = [&](int j, const Idx& ix, int buf) __attribute__((always_inline)) {
+    if (j < RPW) {
+      // row base, chunk permutation and lane in one VALU op (disjoint bits); the empty asm keeps
+      // the address arithmetic at this point of the chain
+      uint32_t base = (uint32_t)__builtin_amdgcn_readlane(ix.nope, j) * (D * 2) + w2::swz(j & 15) * 16;
+      asm volatile("" : "+s"(base));
+      lds_dma16_sbase_untracked(kb, base ^ (uint32_t)(lane * 16), nope_buf[buf] + (wave * RPW + j) * (D * 2));
+    } else {
+      int rid = ix.rope[j - RPW];
+      asm volatile("" : "+v"(rid));
+      const uint16_t* src = (uint32_t)rid < (uint32_t)krows ? krb + (int64_t)rid * DR : ws.zero + 512;
+      lds_dma16_untracked(src + (lane >> 3) * 8, rope_buf[buf] + (wave * RG + j - RPW) * 1024);
+    }
+  };
+
+  // ---- prologue: ids, Q, the first tile's gathers
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (!early_ids || (t + 1) * BN > ws.tstride) ids_dma(t);
+  wait_vmcnt<0>();
+  asm volatile("" ::: "memory");
+  // padded heads are zero; a negative scale runs on the negated query (see sfa_attn_kernel)
+  const uint32_t neg = a.scale < 0.f ? 0x80008000u : 0u;
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const uint8_t* row = &nope_buf[0][0] + (wave * 32 + 16 * n + l16) * (D * 2);
+#pragma unroll
+    for (int j = 0; j < KSN; ++j) qf[j][n] = *reinterpret_cast<const uint4*>(row + (((4 * j + g4) ^ l16) * 16));
+    const bool real = wave * 32 + 16 * n + l16 < n1;
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+      qf[j][n].x = real ? qf[j][n].x ^ neg : 0u;
+      qf[j][n].y = real ? qf[j][n].y ^ neg : 0u;
+      qf[j][n].z = real ? qf[j][n].z ^ neg : 0u;
+      qf[j][n].w = real ? qf[j][n].w ^ neg : 0u;
+    }
+  }
+  lds_barrier();   // every wave's staging reads done, every wave's ids landed
+  uint32_t zero_rows;   // of the tile whose gathers were issued last
+  Idx ix = tile_idx(0);
+  zero_rows = ix.zero_rows;
+#pragma unroll
+  for (int j = 0; j < GPW - 1; ++j) gather_part(j, ix, 0);
+  ix = tile_idx(1);
+
+  float m_used = -INFINITY, m_true = -INFINITY, l_part = 0.f;
+  {
+    float agpr_hint = 0.f;   // O in AGPRs (see sfa_attn_kernel)
+    asm volatile("" : "+a"(agpr_hint));
+  }
+  constexpr int ON = D / 32;
+  f32x16 o[ON];
+#pragma unroll
+  for (int nt = 0; nt < ON; ++nt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[nt][i] = 0.f;
+
+  // LDS addresses in buffer 0, the lane-dependent part. S^T operand (token 16 half + lane % 16, chunk
+  // 4 ks + lane / 16) of k-step ks = 4 a + b at ka[b] + 256 a + 16 rows half; its rope at kr + 512 (ks - 16)
+  // + 2 groups half; V^T operand of columns 32 nt .. + 32, nt = 4 a + b, tokens 8 (lane / 32) + (lane % 16) / 4
+  // at vlo[b] + 256 a and + 4 tokens at vhi[b] + 256 a, 16 rows on for the second half
+  uint32_t ka[4], vlo[4], vhi[4];
+  const uint32_t nb0 = lds_addr(&nope_buf[0][0]);
+  {
+    const int tok = kg * 8 + (l16 >> 2), low = (g4 & 1) * 2 + ((l16 & 3) >> 1);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      ka[b] = nb0 + l16 * (D * 2) + (((4 * b + g4) ^ w2::swz(l16)) * 16);
+      vlo[b] = nb0 + tok * (D * 2) + (((4 * b + low) ^ w2::swz(tok)) * 16) + (l16 & 1) * 8;
+      vhi[b] = nb0 + (tok + 4) * (D * 2) + (((4 * b + low) ^ w2::swz(tok + 4)) * 16) + (l16 & 1) * 8;
+      asm volatile("" : "+v"(ka[b]), "+v"(vlo[b]), "+v"(vhi[b]));
+    }
+  }
+  uint32_t kr = lds_addr(&rope_buf[0][0]) + (l16 >> 3) * 1024 + (g4 * 8 + (l16 & 7)) * 16;
+  asm volatile("" : "+v"(kr));
+  typedef __attribute__((address_space(3), aligned(16))) u32x4v lds_u32x4;
+  auto k_frag = [&](int half, int ks, int buf) __attribute__((always_inline)) -> uint4 {
+    const uint32_t p = ks < KSN ? ka[ks & 3] + (ks >> 2) * 256 + half * 16 * (D * 2) + buf * w2::NOPE
+                                : kr + (ks - KSN) * 512 + half * 2048 + buf * w2::ROPE;
+    const u32x4v v = *(const lds_u32x4*)(uintptr_t)p;
+    return __builtin_bit_cast(uint4, v);
+  };
+  constexpr int NPV = 2 * ON;   // PV MFMAs per tile
+  auto v_frag = [&](int m, int buf) __attribute__((always_inline)) -> uint4 {
+    const int nt = m % ON, off = (m / ON) * 16 * (D * 2) + (nt >> 2) * 256 + buf * w2::NOPE;
+    const uint2 lo = ds_read_tr_at(vlo[nt & 3] + off);
+    const uint2 hi = ds_read_tr_at(vhi[nt & 3] + off);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  };
+
+  constexpr int VR = 6;     // V^T operands in flight
+  constexpr int NPRE = 6;   // PV MFMAs of a tile left for after the next barrier (their operands are read before it)
+  constexpr int KPF = 5;    // S^T operands in flight
+  static_assert(NPRE <= VR && NPRE <= ON && GPW <= 2 * KS, "deferred PV; at most one load per step");
+  uint4 vb[VR];
+  uint4 pb[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};   // P^T B operands of the tile's halves
+#pragma unroll
+  for (int m = 0; m < VR; ++m) vb[m] = make_uint4(0, 0, 0, 0);   // the first tile's deferred MFMAs add zeros
+  auto pv = [&](int m) __attribute__((always_inline)) { o[m % ON] = Mfma<IO>::m32(vb[m % VR], pb[m / ON], o[m % ON]); };
+  float alpha = 1.f, sm_mb = 0.f, sm_mx = 0.f, sm_sum = 0.f;
+  float sc[8];   // raw scores of a half: the lane's head, tokens 8 (lane / 32) + j
+  // Stage st of the online softmax of a half, a few VALU ops each: 0 lanes l and l + 16 trade head tiles, so
+  // that the lane holds 8 tokens of head lane % 32; 1 the max and the exponent reference; 2-5 two
+  // exponentials each, into pb[half]
+  constexpr int NST = 6;
+  auto smx = [&](int st, int half, int t, f32x4& c0, f32x4& c1) __attribute__((always_inline)) {
+    if (st == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sc[i] = c0[i];
+        sc[4 + i] = c1[i];
+        swap_rows16(sc[i], sc[4 + i]);
+      }
+      const int nvalid = ntok - t * BN - half * 16;
+      if (nvalid < 16)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sc[j] = kg * 8 + j < nvalid ? sc[j] : -INFINITY;
+    } else if (st == 1) {
+      sm_mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+      // a half past the row's tokens leaves the reference alone (its max is -inf; a tile's first half holds a token)
+      const float mx = max_half_swap(sm_mx) * cpos;
+      m_true = fmaxf(m_true, mx);
+      const float m_new = mx > m_used + lazy_tau<IO>() ? mx : m_used;
+      alpha = m_used == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_used - m_new) * LOG2E);
+      m_used = m_new;
+      sm_mb = m_used * LOG2E;
+      sm_sum = 0.f;
+    } else {
+      const int i = 2 * (st - 2);
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], cl2, -sm_mb));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i + 1], cl2, -sm_mb));
+      sm_sum += p0;
+      sm_sum += p1;
+      const uint32_t d = pack2<IO>(p0, p1);
+      if (i == 0) pb[half].x = d;
+      else if (i == 2) pb[half].y = d;
+      else if (i == 4) pb[half].z = d;
+      else {
+        pb[half].w = d;
+        l_part = l_part * alpha + sm_sum;
+      }
+    }
+  };
+  auto rescale = [&]() __attribute__((always_inline)) {   // rare (lazy rescaling)
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
+#pragma unroll
+      for (int nt = 0; nt < ON; ++nt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[nt][i] = agpr_scale(o[nt][i], alpha);
+    }
+  };
+
+  // ---- tile t from buffer BUF = t % 2
+  auto tile_body = [&](auto bufc, int t) __attribute__((always_inline)) {
+    constexpr int BUF = decltype(bufc)::value;
+    if (t == 0) wait_vmcnt<0>(); else wait_vmcnt<1>();   // this wave's gathers of tile t
+    if (zero_rows) {   // rare: rows out of range read as zeros
+      wait_vmcnt<0>();
+#pragma unroll 1
+      for (int j = 0; j < RPW; ++j)
+        if ((zero_rows >> j) & 1u)
+          *reinterpret_cast<uint4*>(nope_buf[BUF] + (wave * RPW + j) * (D * 2) + lane * 16) = make_uint4(0, 0, 0, 0);
+    }
+    lds_barrier();   // tile t resident; every wave's reads of tile t-1 done, so its buffer is free
+    f32x4 c[2][2];   // S^T [half][head tile]
+    uint4 af[KPF];
+#pragma unroll
+    for (int j = 0; j < KPF; ++j) af[j] = k_frag(0, j, BUF);
+#pragma unroll
+    for (int m = NPV - NPRE; m < NPV; ++m) pv(m);   // of tile t-1
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, 2 * KS>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value, half = j / KS, ks = j % KS;
+      if constexpr (ks == 0) mfma16x2_vacc_first<IO>(c[half][0], c[half][1], af[j % KPF], qf[ks][0], qf[ks][1]);
+      else if constexpr (ks < KS - 1) mfma16x2_vacc<IO, false>(c[half][0], c[half][1], af[j % KPF], qf[ks][0], qf[ks][1]);
+      else mfma16x2_vacc<IO, true>(c[half][0], c[half][1], af[j % KPF], qf[ks][0], qf[ks][1]);
+      if constexpr (j + KPF < 2 * KS) af[j % KPF] = k_frag((j + KPF) / KS, (j + KPF) % KS, BUF);
+      else if constexpr (j + KPF - 2 * KS < VR) vb[j + KPF - 2 * KS] = v_frag(j + KPF - 2 * KS, BUF);
+      constexpr int g = (j * GPW + 2 * KS - 1) / (2 * KS);   // the load scheduled at this step, if any
+      if constexpr (g < GPW && g * 2 * KS / GPW == j) {
+        if constexpr (g < GPW - 1) gather_part(g, ix, BUF ^ 1);
+        else ids_dma(t + 4);   // slot t % 4 held the ids of tile t, read two iterations ago
+      }
+      if constexpr (half == 1 && (ks & 1) && ks / 2 < NST) smx(ks / 2, 0, t, c[0][0], c[0][1]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    zero_rows = ix.zero_rows;
+#pragma unroll
+    for (int m = KPF; m < VR; ++m) vb[m] = v_frag(m, BUF);
+    rescale();
+    static_for<0, ON>([&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = decltype(mc)::value;
+      pv(m);
+      vb[m % VR] = v_frag(m + VR, BUF);
+      if constexpr ((m & 1) && m / 2 < NST) smx(m / 2, 1, t, c[1][0], c[1][1]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    ix = tile_idx(t + 2);
+    rescale();
+#pragma unroll
+    for (int m = ON; m < NPV - NPRE; ++m) {
+      pv(m);
+      if (m + VR < NPV) vb[m % VR] = v_frag(m + VR, BUF);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    tile_body(std::integral_constant<int, 0>{}, t);
+    if (t + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, t + 1);
+  }
+#pragma unroll
+  for (int m = NPV - NPRE; m < NPV; ++m) pv(m);
+  wait_vmcnt<0>();   // the last (unused) gathers land before the LDS is released
+
+  // ---- epilogue (see sfa_attn_kernel)
+  const float l_tot = l_part + __shfl_xor(l_part, 32);   // l > 0: a row or split holds at least one token
+  if (lane < 32 && hq < n1) {
+    if (direct) {
+      if (a.sm_max) {
+        a.sm_max[(int64_t)r * n1 + hq] = m_true;
+        a.sm_sum[(int64_t)r * n1 + hq] = l_tot * exp2f((m_used - m_true) * LOG2E);
+      }
+    } else {
+      float* ps = ws.part_s + (((int64_t)r * splits + sp) * n1 + hq) * 3;
+      ps[0] = m_used;
+      ps[1] = m_true;
+      ps[2] = l_tot;
+    }
+  }
+  const float inv = 1.f / l_tot;
+  const int hc = min(hq, n1 - 1);
+  uint16_t* orow = (direct ? out + ((int64_t)r * n1 + hc) * D : ws.part_o + (((int64_t)r * splits + sp) * n1 + hc) * D) +
+                   kg * 8;
+#pragma unroll
+  for (int nt = 0; nt < ON; ++nt) {
+    uint32_t d[4][2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      d[g][0] = pack2<IO>(o[nt][4 * g] * inv, o[nt][4 * g + 1] * inv);
+      d[g][1] = pack2<IO>(o[nt][4 * g + 2] * inv, o[nt][4 * g + 3] * inv);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      swap_halves(d[0][j], d[1][j]);
+      swap_halves(d[2][j], d[3][j]);
+    }
+    if (hq < n1) {
+      stg16(orow + nt * 32, make_uint4(d[0][0], d[0][1], d[1][0], d[1][1]));
+      stg16(orow + nt * 32 + 16, make_uint4(d[2][0], d[2][1], d[3][0], d[3][1]));
+    }
+  }
+}
+
 // ---------------------------------------------------------------- kernel 2, 64-head form (D = 512)
 // One work-group of 8 waves (two per SIMD) per (query row, 64 heads, KV split), launched
-// for N1 <= 64 (the reference's perf_sfa shape). O^T and Q^T of 64 heads take half the
+// for N1 <= 64 where the work-groups number at most one a CU (see launch_attn_d). O^T and Q^T of 64 heads take half the
 // registers of the 128-head form, so two waves share each SIMD.
 //  * S^T[32 tokens, 32 heads] of head block hb = w % 2 is split over the contraction:
 //    wave w runs k-steps [9 q, 9 q + 9), q = w / 2 (Q^T fragments of those k-steps, rope
@@ -1489,9 +1889,6 @@ __global__ __launch_bounds__(NWV * 64) void sfa_attn_kernel(SfaArgs a, int cap, 
 //  * Gathers: wave w copies the nope rows of tokens 4w .. 4w + 3, waves 0-3 the rope of
 //    tokens 8w .. 8w + 7, every wave its 4 ids of the tile four ahead (the last load of
 //    an iteration, so one vmcnt wait retires a tile in every wave).
-//  * Rows of more than 64 heads would run as two halves launched 8 work-groups apart
-//    (round-robin dispatch over the 8 XCDs puts them on one XCD, whose L2 then serves
-//    both halves' gathers); the launcher keeps such rows on the 128-head form.
 namespace w8 {
 constexpr int NW = 8;          // waves
 constexpr int HH = 64;         // heads per work-group
@@ -1515,13 +1912,7 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   __shared__ float s_alpha[w8::HH];   // O rescale factors (rare path)
   __shared__ int s_flag[2];           // a group exceeded m_used + TAU, by tile parity
 
-  // (row, head half, split) of this work-group; halves of one (row, split) 8 apart
-  const int nh = a.n1 > w8::HH ? 2 : 1;
-  const int nq = a.total_rows * splits;
-  const int x = blockIdx.x;
-  const int q = nh == 2 ? (x >> 4) * 8 + (x & 7) : x;
-  const int hh = nh == 2 ? (x >> 3) & 1 : 0;
-  if (q >= nq) return;
+  const int q = blockIdx.x;   // (row, split)
   const int sp = q / a.total_rows;
   const int r = a.total_rows - 1 - (q - sp * a.total_rows);   // long (late causal) rows first
 
@@ -1529,7 +1920,7 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hb = wave_u & 1, kq = wave_u >> 1;
   const int n1 = a.n1;
-  const int h0 = hh * w8::HH;
+  constexpr int h0 = 0;
   const int hl = hb * 32 + (lane & 31);   // local head of this lane's S^T column
   const int hs = h0 + hl;
   const int ntok_all = ws.counts[r];
@@ -1873,17 +2264,21 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
 
 template <int IO, int D>
 hipError_t launch_attn_d(const SfaArgs& a, hipStream_t s, int cap, int splits, int fuse_tok, Ws ws) {
-  // N1 <= 64: the 8-wave form (one work-group per row). Above 64 heads the 128-head form:
-  // split into two 64-head work-groups a row pays two serial prologues and its tiles run
-  // at about 1.5x the 128-head form's cycles (measured), so it stays one work-group.
-  if (D == w8::DD && !fuse_tok && a.n1 <= w8::HH) {   // token lists built by the token-list launch
-    const int64_t nq = (int64_t)a.total_rows * splits;
-    const int64_t grid = a.n1 > w8::HH ? (nq + 7) / 8 * 16 : nq;
-    hipLaunchKernelGGL(sfa_attn8_kernel<IO>, dim3((unsigned)grid), dim3(w8::NW * 64), 0, s, a, splits, ws);
+  // Both per-wave forms gather with 32-bit row offsets. With N1 <= 64, D = 512 and token lists from
+  // the token-list launch: the two-wave form, whose work-groups share a CU by twos (4026 packed rows of
+  // 64 heads, fp16, 808 -> 585 us; 32 heads 763 -> 523; 300 rows of 2048 tokens 206 -> 145), unless there is
+  // at most one a CU: then eight waves on a row (256 rows 124 us against 154). Above 64 heads one
+  // work-group of four waves per row: two of the two-wave form would gather every row twice.
+  const bool off32 = (uint64_t)a.key_rows * D * 2 <= (1ull << 32);
+  const int64_t nq = (int64_t)a.total_rows * splits;
+  if (D == w2::D && !fuse_tok && a.n1 <= w2::NW * 32 && off32 && nq > 256) {
+    hipLaunchKernelGGL(sfa_attn2_kernel<IO>, dim3(a.total_rows, splits), dim3(w2::NW * 64), 0, s, a, splits, ws);
+  } else if (D == w8::DD && !fuse_tok && a.n1 <= w8::HH) {
+    hipLaunchKernelGGL(sfa_attn8_kernel<IO>, dim3((unsigned)nq), dim3(w8::NW * 64), 0, s, a, splits, ws);
   } else if (a.n1 <= 64)
     hipLaunchKernelGGL((sfa_attn_kernel<IO, D, 64, false>), dim3(a.total_rows, splits), dim3(NWV * 64), 0, s, a,
                        cap, splits, fuse_tok, ws);
-  else if ((uint64_t)a.key_rows * D * 2 <= (1ull << 32))   // its gathers use 32-bit row offsets
+  else if (off32)
     hipLaunchKernelGGL((sfa_attn_kernel<IO, D, 128, false, true>), dim3(a.total_rows, splits), dim3(NWV * 64), 0, s,
                        a, cap, splits, fuse_tok, ws);
   else

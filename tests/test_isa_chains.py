@@ -1,5 +1,5 @@
 """The SFA forward's S^T chains are inline-asm MFMAs with VGPR accumulators
-(dsa_common.hpp: mfma32_vacc*). The compiler does not know those MFMAs are in flight,
+(dsa_common.hpp: mfma32_vacc*, mfma16x2_vacc*). The compiler does not know those MFMAs are in flight,
 so it could copy or reuse an accumulator register between two steps of a chain (or
 before its drain) and read a result that is not there yet: a silent wrong answer that a
 GPU test sees only on the shapes where the register allocation happens to do it.
@@ -19,7 +19,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 SRC = os.path.join(ROOT, "dsa_triton_ascend_amd", "csrc", "sfa_fwd.hip")
 DRAIN = 18   # wait states after the last MFMA of a chain (dsa_common.hpp: vacc_drain)
 
-_MFMA = re.compile(r"\s*v_mfma_f32_32x32x16_(?:bf16|f16) v\[(\d+):(\d+)\], (v\[\d+:\d+\]), (v\[\d+:\d+\]), (\S+)")
+_MFMA = re.compile(r"\s*v_mfma_f32_(?:32x32x16|16x16x32)_(?:bf16|f16) v\[(\d+):(\d+)\], (v\[\d+:\d+\]), (v\[\d+:\d+\]), (\S+)")
 
 
 def _regs(text):

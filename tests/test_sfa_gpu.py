@@ -495,3 +495,43 @@ def test_workspace_contents_past_zero_prefix_are_ignored(dev, fill):
             out, smax, ssum = plan.run()
             torch.cuda.synchronize()
             compare(out, smax, ssum, *o, what=f"workspace fill {fill} kv_splits={kv_splits} call {rep}")
+
+
+@pytest.mark.parametrize("N1,dtype,scale", [(64, "bf16", 0.04), (64, "fp16", -0.04), (16, "fp16", 0.04)])
+def test_two_wave_form_rows_of_every_length(dev, N1, dtype, scale):
+    """D = 512, at most 64 heads, more rows than CUs (two waves a row): 300 causal rows of 1 .. 70
+    tokens, so every remainder of the 16-token halves and the 32-token tiles, over a paged cache
+    with a missing page (zero key rows) and a row without tokens."""
+    B, S, D, count, page = 1, 300, 512, 70, 16
+    q, k, _, qr, kr = _inputs(B, S, 320, N1, D, dtype, seed=21)
+    si = _ref_indices(B, S, S, count, 1, 3, seed=22)
+    si[0, 40, 0, :] = -1
+    bt = np.random.RandomState(23).permutation(20).astype(np.int32)[None, :]
+    cache, rcache = k.reshape(20, page, 1, D), kr.reshape(20, page, 1, 64)
+    bt[0, 3] = -1
+    kw = dict(scale_value=scale, actual_seq_lengths_kv=[S], sparse_mode=3, return_softmax_lse=True,
+              layout_kv="PA_BSND", block_size=page)
+    out, smax, ssum = sparse_flash_attention(q.to(dev), cache.to(dev), cache.to(dev), torch.from_numpy(si).to(dev),
+                                             block_table=torch.from_numpy(bt).to(dev), query_rope=qr.to(dev),
+                                             key_rope=rcache.to(dev), **kw)
+    torch.cuda.synchronize()
+    o = SFA.sparse_flash_attention(_np(q), _np(cache), None, si, block_table=bt, query_rope=_np(qr),
+                                   key_rope=_np(rcache), io_dtype=dtype, **kw)
+    compare(out, smax, ssum, *o, what=f"two-wave N1={N1} {dtype} scale={scale}")
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_two_wave_form_climbing_scores(dev, dtype):
+    """The two-wave form's lazy rescaling, moved several times a row (see test_climbing_score_spread)."""
+    S1, N1, D = 4, 64, 512
+    q, k, qr, kr, scale = _climbing_inputs(S1, N1, D, dtype, (35.0, 15.0, 22.0))
+    si = np.tile(np.arange(256, dtype=np.int32), (1, S1, 1, 1))
+    o = SFA.sparse_flash_attention(_np(q), _np(k), None, si, scale, query_rope=_np(qr), key_rope=_np(kr),
+                                   sparse_mode=0, return_softmax_lse=True, io_dtype=dtype)
+    rep = lambda t: t.repeat(1, 70, 1, 1).to(dev)   # 280 rows: the same four again and again
+    out, smax, ssum = sparse_flash_attention(rep(q), k.to(dev), k.to(dev), rep(torch.from_numpy(si)), scale_value=scale,
+                                             query_rope=rep(qr), key_rope=kr.to(dev), sparse_mode=0,
+                                             return_softmax_lse=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :4], out[:, -4:]) and torch.equal(out[:, :4], out[:, 140:144])
+    compare(out[:, :4], smax[:, :, :4], ssum[:, :, :4], *o, what=f"two-wave climbing {dtype}")
