@@ -2,6 +2,8 @@
 dtype codes, stream handles and the small int32 index arrays the C ABI takes."""
 from __future__ import annotations
 
+from array import array
+
 import torch
 
 from . import _lib
@@ -74,12 +76,39 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
-def i32(values: list[int], device: torch.device) -> torch.Tensor:
-    return torch.tensor(values, dtype=torch.int32).to(device, non_blocking=True)
+UPLOAD_MAX = 8192   # dsa_upload_i32's limit
+
+
+def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | None = None):
+    """The int32 length and offset arrays of a call on the device, views of one tensor (each padded
+    to 16 bytes), written by one launch on the current stream (dsa_upload_i32); `zero` (a
+    byte tensor) is cleared by the same launch. More values than a launch takes, or a device
+    that is not the current one, go by a copy."""
+    flat, sizes = array("i"), []
+    try:
+        for a in arrays:
+            flat.extend(a)
+            pad = -len(flat) % 4
+            if pad:
+                flat.extend((0,) * pad)
+            sizes.append(len(a) + pad)
+    except OverflowError as e:   # torch's error for such a value
+        raise RuntimeError("value cannot be converted to type int32 without overflow") from e
+    n = len(flat)
+    if n <= UPLOAD_MAX and device.index in (None, torch.cuda.current_device()):
+        t = torch.empty(n, dtype=torch.int32, device=device)
+        _lib.check(lib.dsa_upload_i32(flat.buffer_info()[0], n, t.data_ptr(), ptr(zero),
+                                      0 if zero is None else zero.numel(), stream_ptr(device)), "dsa_upload_i32")
+    else:
+        t = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=True)
+        if zero is not None:
+            zero.zero_()
+    return t.split(sizes)
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle, without the Stream object that torch.cuda.current_stream builds (2.5 us a call)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -28,6 +28,7 @@ _F = ctypes.c_float
 SIGNATURES = {
     "dsa_abi_version": (_I, []),
     "dsa_last_error": (ctypes.c_char_p, []),
+    "dsa_upload_i32": (_I, [_P, _I, _P, _P, _SZ, _P]),
     "dsa_li_score": (_I, [_P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I,
                           _P, _I64, _P]),
     "dsa_li_topk": (_I, [_P, _I64, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P]),

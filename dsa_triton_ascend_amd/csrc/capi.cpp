@@ -37,6 +37,24 @@ int hip_status(hipError_t e, const char* what) {
 }
 
 bool is16(int dt) { return dt == DSA_DTYPE_BF16 || dt == DSA_DTYPE_F16; }
+
+// A call's length and offset arrays travel as kernel arguments. A copy from pageable memory made the
+// host wait for the stream (four of them a call: about 20 us in which the GPU idled between calls).
+constexpr int UPLOAD_MAX = 8192;   // ints per call
+template <int N> struct UploadArgs { int32_t v[N]; };
+
+template <int N>
+__global__ __launch_bounds__(256) void upload_i32_kernel(UploadArgs<N> a, int n, int32_t* dst, uint4* zero, int n16) {
+  for (int i = threadIdx.x; i < n; i += 256) dst[i] = a.v[i];
+  for (int i = threadIdx.x; i < n16; i += 256) zero[i] = make_uint4(0, 0, 0, 0);
+}
+
+template <int N>
+void launch_upload(const int32_t* host, int n, int32_t* dst, void* zero, int n16, hipStream_t s) {
+  UploadArgs<N> a;
+  std::memcpy(a.v, host, sizeof(int32_t) * (size_t)n);
+  hipLaunchKernelGGL(upload_i32_kernel<N>, dim3(1), dim3(256), 0, s, a, n, dst, reinterpret_cast<uint4*>(zero), n16);
+}
 }  // namespace
 
 extern "C" {
@@ -44,6 +62,30 @@ extern "C" {
 int dsa_abi_version(void) { return 1; }
 
 const char* dsa_last_error(void) { return g_err; }
+
+int dsa_upload_i32(const int32_t* host, int n, int32_t* dst, void* zero_dst, size_t zero_bytes, void* stream) {
+  if (n < 0 || (n > 0 && (!host || !dst)))
+    return fail(DSA_ERR_INVALID, "dsa_upload_i32: null pointer argument or negative count");
+  if (n > UPLOAD_MAX) return fail(DSA_ERR_UNSUPPORTED, "dsa_upload_i32: n=%d > %d", n, UPLOAD_MAX);
+  if (!zero_dst) zero_bytes = 0;
+  if (zero_bytes % 16 != 0 || zero_bytes > (1 << 20) || ((uintptr_t)zero_dst & 15) != 0)
+    return fail(DSA_ERR_INVALID, "dsa_upload_i32: zero_dst / zero_bytes must be multiples of 16, at most 1 MiB");
+  const hipStream_t s = (hipStream_t)stream;
+  const int n16 = (int)(zero_bytes / 16);
+  if (n == 0 && n16 == 0) {
+    g_err[0] = 0;
+    return DSA_OK;
+  }
+  // kernel arguments are limited to 4 KiB; most calls fit the small form
+  constexpr int SMALL = 56, LARGE = 960;
+  if (n <= SMALL) {
+    launch_upload<SMALL>(host, n, dst, zero_dst, n16, s);
+  } else {
+    for (int i = 0; i < n; i += LARGE)
+      launch_upload<LARGE>(host + i, n - i < LARGE ? n - i : LARGE, dst + i, zero_dst, i == 0 ? n16 : 0, s);
+  }
+  return hip_status(hipGetLastError(), "dsa_upload_i32 launch");
+}
 
 int dsa_li_score(const void* query, const void* key, const void* weights, int io_dtype,
                  int w_dtype, const int32_t* row_start, const int32_t* key_start,

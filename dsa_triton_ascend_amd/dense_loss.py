@@ -75,7 +75,7 @@ def dense_lightning_indexer_softmax_lse(query_index, key_index, weights, actual_
     wdt = H.dtype_code(weights.dtype, "weights", allow_f32=True)
     B, S1, Nidx1, Didx = query_index.shape
     S2 = key_index.shape[1]
-    act_q, act_k = H.i32(aq, dev), H.i32(ak, dev)
+    act_q, act_k = H.upload(lib, dev, aq, ak)
     qi, ki, w = query_index.contiguous(), key_index.contiguous(), weights.contiguous()
     mx = torch.empty((B, 1, S1), dtype=torch.float32, device=dev)
     sm = torch.empty((B, 1, S1), dtype=torch.float32, device=dev)
@@ -165,7 +165,7 @@ class DenseLossPlan:
         self.loss = torch.empty(1, dtype=torch.float32, device=dev)
         self.ws_bytes = lib.dsa_dense_li_grad_workspace_bytes(B, S1, S2, Didx)
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.d_aq, self.d_ak = H.i32(aq, dev), H.i32(ak, dev)
+        self.d_aq, self.d_ak = H.upload(lib, dev, aq, ak)
         self.lib, self.dev = lib, dev
         self.io = H.dtype_code(query.dtype, "query")
         self.wdt = H.dtype_code(weights.dtype, "weights", allow_f32=True)

@@ -108,10 +108,8 @@ class IndexerPlan:
         self.scores = torch.empty((max(total_rows, 1) * N2, self.ld), dtype=torch.int16, device=dev)
         tw = int(self.lib.dsa_li_topk_workspace_bytes(total_rows, N2, S2, self.k))
         self.topk_ws = torch.empty(tw, dtype=torch.uint8, device=dev) if tw > 0 else None
-        self.d_row_start = H.i32(row_start, dev)
-        self.d_key_start = H.i32(key_start, dev)
-        self.d_aq = H.i32(act_q, dev)
-        self.d_ak = H.i32(act_k, dev)
+        self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(self.lib, dev, row_start, key_start,
+                                                                            act_q, act_k)
         self.max_rows = max(row_start[b + 1] - row_start[b] for b in range(B)) if B else 0
         self.max_kv = max(act_k) if act_k else 0
 

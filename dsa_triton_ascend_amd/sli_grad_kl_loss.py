@@ -105,7 +105,7 @@ class KLLossPlan:
         self.loss = torch.empty(1, dtype=torch.float32, device=dev)
         self.ws_bytes = lib.dsa_sli_grad_workspace_bytes(B, S1, S2, topk, Didx)
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.d_aq, self.d_ak = H.i32(act_q, dev), H.i32(act_k, dev)
+        self.d_aq, self.d_ak = H.upload(lib, dev, act_q, act_k)
         self.lib, self.io, self.wdt, self.dev = lib, io, wdt, dev
         self.dims = (B, S1, S2, N1, D, Dr, Nidx1, Didx, topk)
         self.scale = float(scale_value)

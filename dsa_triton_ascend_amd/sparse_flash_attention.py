@@ -143,11 +143,9 @@ class AttentionPlan:
         # the workspace starts with a zero KV row that the library keeps at zero across
         # calls; only that prefix needs clearing (include/dsa_mi355x.h, dsa_sfa_fwd)
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.ws[:min(self.ws.numel(), lib.dsa_sfa_workspace_zero_bytes())].zero_()
-        self.d_row_start = H.i32(row_start, dev)
-        self.d_key_start = H.i32(key_start, dev)
-        self.d_aq = H.i32(act_q, dev)
-        self.d_ak = H.i32(act_k, dev)
+        zero = self.ws[:lib.dsa_sfa_workspace_zero_bytes()] if self.ws_bytes else None
+        self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(lib, dev, row_start, key_start, act_q,
+                                                                            act_k, zero=zero)
         self.act_q, self.act_k, self.row_start = act_q, act_k, row_start
         self.key_rows = kk.numel() // D
 
@@ -163,8 +161,8 @@ class AttentionPlan:
                 self.out.data_ptr(), H.ptr(self.sm_max), H.ptr(self.sm_sum), self.ws.data_ptr(),
                 self.ws_bytes, self.kv_splits, H.stream_ptr(self.dev)), "dsa_sfa_fwd")
         if not self.return_lse:
-            z = torch.zeros(self.sm_shape, dtype=torch.float32, device=self.dev)
-            return self.out, z, z.clone()
+            z = torch.zeros((2,) + self.sm_shape, dtype=torch.float32, device=self.dev)
+            return self.out, z[0], z[1]
         return self.out, self.sm_max, self.sm_sum
 
 

@@ -134,10 +134,8 @@ class GradPlan:
         if self.ws_bytes == 0:
             raise ValueError("dsa_sfa_bwd_workspace_bytes rejected the shapes")
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.d_row_start = H.i32(row_start, dev)
-        self.d_key_start = H.i32(key_start if key_start else [0], dev)
-        self.d_aq = H.i32(act_q, dev)
-        self.d_ak = H.i32(act_k, dev)
+        self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(lib, dev, row_start, key_start or [0],
+                                                                            act_q, act_k)
 
     def run(self):
         _lib.check(self.lib.dsa_sfa_bwd(

@@ -56,6 +56,16 @@ int dsa_abi_version(void);
 const char* dsa_last_error(void);
 
 /*
+ * Copies n int32 values from host memory to device memory on `stream`, as kernel
+ * arguments: the host neither waits for the stream nor needs `host` to outlive the call,
+ * and the call may be captured (the values are then part of the graph). Also clears
+ * zero_bytes (a multiple of 16) at zero_dst, 16-byte aligned, if zero_dst is not NULL. For
+ * the small length and offset arrays the entry points below take; n <= 8192
+ * (DSA_ERR_UNSUPPORTED above: use a copy). No counterpart in the reference.
+ */
+int dsa_upload_i32(const int32_t* host, int n, int32_t* dst, void* zero_dst, size_t zero_bytes, void* stream);
+
+/*
  * Indexer scores (replaces _lightning_indexer_score_core,
  * lightning_indexer_triton.py:386-417).
  *

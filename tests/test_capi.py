@@ -317,3 +317,35 @@ def test_grad_rejects_decreasing_host_row_start():
                          ctypes.cast(ak, ctypes.c_void_p), 3, 8, 8, 128, 64, 64, 192, 3, 0.1, p, p, p, p,
                          p, p, p, p, p, p, 1 << 30, None)
     assert st == _lib.DSA_ERR_INVALID and b"non-decreasing" in lib.dsa_last_error()
+
+
+def test_upload_i32_rejects_bad_arguments():
+    lib = _lib.load()
+    assert lib.dsa_upload_i32(None, 3, None, None, 0, None) == _lib.DSA_ERR_INVALID
+    buf = (ctypes.c_int32 * 4)()
+    p = ctypes.cast(buf, ctypes.c_void_p)
+    assert lib.dsa_upload_i32(p, -1, p, None, 0, None) == _lib.DSA_ERR_INVALID
+    assert lib.dsa_upload_i32(p, 8193, p, None, 0, None) == _lib.DSA_ERR_UNSUPPORTED
+    assert lib.dsa_upload_i32(p, 4, p, 16, 24, None) == _lib.DSA_ERR_INVALID
+    assert lib.dsa_upload_i32(p, 0, None, None, 0, None) == _lib.DSA_OK   # nothing to do: no launch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [(1, 0, 3, 1), (14, 14, 14, 14), (57,), (960,), (961, 2), (8192,), (8193, 5)])
+def test_upload_of_length_arrays(counts):
+    """The call's length arrays at the edges of the launch's sizes (56 and 960 values a launch, 8192
+    a call, a copy above), padded to 16 bytes each, with the workspace prefix cleared beside them."""
+    from dsa_triton_ascend_amd import _host as H
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda:0")
+    arrays = [[(7 * i + 13 * j) % 100003 - 50000 for i in range(n)] for j, n in enumerate(counts)]
+    zero = torch.full((1152,), 255, dtype=torch.uint8, device=dev)
+    guard = torch.full((64,), 255, dtype=torch.uint8, device=dev)
+    got = H.upload(_lib.load(), dev, *arrays, zero=zero)
+    for a, t in zip(arrays, got):
+        assert t.data_ptr() % 16 == 0 or not a
+        assert t[:len(a)].tolist() == a and not t[len(a):].any()
+    assert not zero.any() and bool((guard == 255).all())
+    with pytest.raises(RuntimeError):
+        H.upload(_lib.load(), dev, [1 << 31])
