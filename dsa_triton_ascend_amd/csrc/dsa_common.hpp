@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/dsa_mi355x.h"
 
 namespace dsa {
@@ -17,6 +19,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
 enum IoType { IO_F16 = DSA_DTYPE_F16, IO_BF16 = DSA_DTYPE_BF16 };
 
@@ -171,6 +174,46 @@ __device__ __forceinline__ void mfma16x2_vacc(f32x4& c0, f32x4& c1, uint4 a, uin
 }
 #undef DSA_MFMA16_PAIR
 
+// Two last steps of one chain of such a pair (its own accumulator only), drained.
+template <int IO>
+__device__ __forceinline__ void mfma16_vacc_last2(f32x4& c, uint4 a0, uint4 b0, uint4 a1, uint4 b1) {
+  const i32x4v av0 = __builtin_bit_cast(i32x4v, a0), bv0 = __builtin_bit_cast(i32x4v, b0);
+  const i32x4v av1 = __builtin_bit_cast(i32x4v, a1), bv1 = __builtin_bit_cast(i32x4v, b1);
+  if constexpr (IO == IO_BF16)
+    asm volatile(
+        "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tv_mfma_f32_16x16x32_bf16 %0, %3, %4, %0\n\ts_nop 15\n\ts_nop 1"
+        : "+v"(c) : "v"(av0), "v"(bv0), "v"(av1), "v"(bv1));
+  else
+    asm volatile(
+        "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tv_mfma_f32_16x16x32_f16 %0, %3, %4, %0\n\ts_nop 15\n\ts_nop 1"
+        : "+v"(c) : "v"(av0), "v"(bv0), "v"(av1), "v"(bv1));
+}
+
+// f(integral_constant I), f(I + 1), .. f(N - 1): an unrolled loop whose body may be of any size (the
+// compiler gives up on `#pragma unroll` of very large ones and moves the arrays they index to scratch)
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// Gathered KV rows of 1024 bytes, unpadded in LDS: 16-byte chunk c of token t sits at c ^ kv_swz(t), a
+// bijection of t % 16 chosen for both readers. The 8 consecutive tokens of an operand read (16 tokens,
+// one chunk) differ in its low three bits; the four tokens of a transposed read in bits 2 and 3 and in
+// bits 1 and 2, so their 32- or 64-byte runs lie on distinct banks.
+__host__ __device__ constexpr int kv_swz(int t) {
+  return ((((t >> 1) ^ (t >> 3)) & 1) << 3) | ((t & 1) << 2) | (t & 2) | ((t >> 2) & 1);
+}
+// 16-byte LDS read at a 32-bit LDS address (a typedef that carries the alignment: without it the
+// compiler splits the read)
+typedef __attribute__((address_space(3), aligned(16))) u32x4v lds_u32x4v;
+__device__ __forceinline__ uint4 lds_read16_at(uint32_t lds_addr) {
+  const u32x4v v = *(const lds_u32x4v*)(uintptr_t)lds_addr;
+  return __builtin_bit_cast(uint4, v);
+}
+
 // Output layouts (CDNA3/CDNA4 MFMA, 64 lanes):
 //  32x32: lane l, acc[r] (r < 16) holds C[row = (r/4)*8 + (l/32)*4 + r%4][col = l%32]
 //  16x16: lane l, acc[r] (r < 4)  holds C[row = (l/16)*4 + r][col = l%16]
@@ -184,7 +227,6 @@ __device__ __forceinline__ int m16_row(int r, int lane) { return (lane >> 4) * 4
 // compiler emit flat loads (for instance where it turns `c ? load(p) : zero` into a
 // load from a selected address), and a flat load is counted by lgkmcnt as well, so
 // every later LDS wait would also wait for it.
-typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 ldg16(const void* p) {
   return __builtin_bit_cast(uint4, *(const __attribute__((address_space(1))) u32x4v*)p);
 }

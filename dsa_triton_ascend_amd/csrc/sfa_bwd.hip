@@ -72,7 +72,7 @@ constexpr int BWV = 8;      // waves per work-group (two per SIMD)
 constexpr float BLOG2E = 1.4426950408889634f;
 constexpr int GBK = 64;     // dense rows are padded to a multiple of 64 (row, head) pairs
 constexpr size_t LT_WS = (size_t)128 << 20;  // workspace offered to the library GEMMs
-constexpr int LT_CANDIDATES = 64;            // length of the heuristic's ranked list
+constexpr int LT_CANDIDATES = 4;             // length of the heuristic's ranked list asked for
 // Split of the products' contraction (the batch's (row, head) pairs): with M = key rows
 // and N = D + Dr or D the output has few tiles (about 64 - 144 at the grad perf shape for
 // 256 CUs), so the contraction is cut into BSPLIT chunks, run as one strided-batched
@@ -122,6 +122,7 @@ struct BwdWs {
   uint16_t* pt;    // P_T dense buffer (io dtype)
   int64_t cap;     // elements per dense buffer
   int zfuse;       // the rows kernel writes the zeros of the dense buffers (no clear kernels)
+  int max_nk;      // key tokens of the longest batch
 };
 
 // Dense geometry of batch b: query rows [rs, rs + nq), key rows [ks, ks + nk)
@@ -134,7 +135,12 @@ struct BatchGeo {
 
 __host__ __device__ inline int batch_nk(int act_k, int s2) { return act_k < 0 ? 0 : (act_k < s2 ? act_k : s2); }
 
-__host__ __device__ inline int dense_row(int nq, int n1) { return (nq * n1 + GBK - 1) / GBK * GBK; }
+// (64 more where the row would be a multiple of 2 KiB: dense rows a power of two apart put a product's
+// column panel on few memory channels; 512 rows of 64 heads over 4096 keys 740 -> 719 us the call)
+__host__ __device__ inline int dense_row(int nq, int n1) {
+  const int r = (nq * n1 + GBK - 1) / GBK * GBK;
+  return r % 1024 == 0 ? r + GBK : r;
+}
 
 __device__ __forceinline__ BatchGeo batch_geo(const SfaArgs& f, int b) {
   BatchGeo g;
@@ -530,6 +536,374 @@ __global__ __launch_bounds__(BWV * 64) void sfa_bwd_rows_kernel(SfaBwdArgs a, Sf
   }
 }
 
+// ---------------------------------------------------------------- rows kernel, 64 heads (D = 512)
+// The rows kernel for N1 a multiple of 64: one work-group of four waves (one per SIMD) per (query row,
+// 64 heads); wave w runs everything of its own 16 heads, so a tile's scores never leave its registers
+// and each gathered row serves 64 heads instead of 32.
+//  * Q | Q rope and dO (136 VGPRs a lane) and dQ^T[576, 16 heads] (144 AGPRs) stay in registers for the row.
+//  * The rows of a 32-token tile are gathered with direct-to-LDS loads two tiles ahead into a ring of four
+//    (chunks permuted by kv_swz); one LDS-only barrier per tile. Tile t runs S^T and dP^T of t, then dQ of
+//    t - 1 with P and dS of t (VALU) among its MFMAs.
+//  * S^T and dP^T share each K operand: 16x16x32 MFMAs with 16 tokens as M and the wave's heads as N, so a
+//    lane holds 4 tokens of one head per half tile -- with the other half's 4 exactly the B operand of
+//    dQ^T += K^T dS^T in the token order {4g + j, 16 + 4g + j}, which the transposed K reads follow.
+//  * P and dS also pass through a 2.5 KB LDS tile of the wave's own, from which transposed reads give each
+//    lane four heads of one token for the dense buffers' stores.
+// 512 rows of 64 heads over 4096 keys, 2048 tokens a row: this kernel 370 us against 560 for the 32-head
+// form (968 -> 719 us the call). Without its stores and gathers it takes 211 us, of which 101 of MFMA
+// at one wave per SIMD; the 536 MB of P, dS and zeros, in runs of 32 to 128 bytes, cost the rest.
+namespace r64 {
+constexpr int D = 512, DT = D + BDR;
+constexpr int NW = 4;                     // waves, 16 heads each
+constexpr int NH = 16 * NW;
+constexpr int KS = DT / 32, KSN = D / 32;   // S^T k-steps (18), of which nope (16)
+constexpr int NBUF = 4;
+constexpr int NOPE = BT * D * 2, ROPE = BT * BDR * 2;
+constexpr int NB = DT / 16;               // 16-column blocks of dQ^T (36)
+constexpr int GPW = BT / NW + 2;          // loads per wave per tile: 8 nope rows, rope, ids
+constexpr int VR = 6;                     // dQ operands in flight
+constexpr int SP = BT + 8;                // pitch of the P / dS tile (elements)
+constexpr int ZBW = 1024;                 // words of the selected-token bitmap (what the LDS has left)
+// rope rows of 128 bytes: 16-byte chunk c of token t at c ^ rswz(t)
+__host__ __device__ constexpr int rswz(int t) { return ((t & 3) << 1) | ((t >> 2) & 1); }
+}  // namespace r64
+
+template <int IO>
+__global__ __launch_bounds__(r64::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void sfa_bwd_rows64_kernel(SfaBwdArgs a, SfaTokenLists tl, BwdWs w) {
+  using namespace r64;
+  __shared__ __attribute__((aligned(1024))) uint8_t nope_buf[NBUF][NOPE];
+  __shared__ __attribute__((aligned(1024))) uint8_t rope_buf[NBUF][ROPE];
+  __shared__ __attribute__((aligned(16))) uint16_t stage[NW][2][16 * SP];   // [P, dS][head][token] of a wave
+  __shared__ __attribute__((aligned(16))) int32_t s_ids[8][BT];   // token-id ring: tile t in slot t % 8
+  __shared__ uint32_t s_sel[ZBW];    // the batch tokens this row writes to the dense buffers
+
+  const SfaArgs& f = a.f;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int r = f.total_rows - 1 - (int)blockIdx.x;   // long (late causal) rows first
+  const int n1 = f.n1;
+  const int h0 = blockIdx.y * NH;
+  const int krows = f.key_rows < INT_MAX ? (int)f.key_rows : INT_MAX;
+  const int ntok = __builtin_amdgcn_readfirstlane(tl.counts[r]);
+  const int32_t* toks = tl.tokens + (int64_t)r * tl.tstride;
+  const uint16_t* kb = reinterpret_cast<const uint16_t*>(f.k);
+  const uint16_t* krb = reinterpret_cast<const uint16_t*>(f.kr);
+  const uint4 z4 = make_uint4(0, 0, 0, 0);
+  const int b = batch_of_row(f.row_start, f.batch, r);
+  const BatchGeo g = batch_geo(f, b);
+  const int rl = r - g.rs;
+  const bool dense_ok = rl >= 0 && rl < g.nq && w.boff[b + 1] <= w.cap;
+  const int64_t dbase = w.boff[b] + (int64_t)rl * n1 + h0;   // (row, head block)'s column of dense row 0
+  const bool zf = w.zfuse && dense_ok;   // the host checked nk <= 32 ZBW
+
+  const int ntiles = (ntok + BT - 1) / BT;
+  auto clamp_tile = [&](int t) { return t < ntiles ? t : ntiles - 1; };
+  // this wave's 8 ids of tile t into the ring (tiles past the end re-read the last)
+  auto ids_dma = [&](int t) {
+    if (lane < 2)
+      lds_dma16_sbase_untracked(toks, (uint32_t)(clamp_tile(t) * BT + wave * 8) * 4 + lane * 16,
+                                &s_ids[0][0] + __builtin_amdgcn_readfirstlane((t & 7) * BT + wave * 8));
+  };
+  if (ntok > 0)
+#pragma unroll
+    for (int t = 0; t < 5; ++t) ids_dma(t);
+
+  // ---- Q | Q rope and dO of head h0 + 16 wave + lane % 16 (8 elements at 32 ks + 8 (lane / 16)), copied to the
+  // products' operands as they pass (zeros for a row without tokens, so that whatever its inputs hold
+  // never reaches d_key / d_value); delta = dO . O
+  const int64_t hr = (int64_t)r * n1 + h0 + wave * 16 + l16;
+  uint4 qf[KS], gf[KSN];
+  float dl = 0.f;
+  {
+    const uint16_t* q = reinterpret_cast<const uint16_t*>(f.q) + hr * D + g4 * 8;
+    const uint16_t* qr = reinterpret_cast<const uint16_t*>(f.qr) + hr * BDR + g4 * 8;
+    const uint16_t* go = reinterpret_cast<const uint16_t*>(a.d_out) + hr * D + g4 * 8;
+    const uint16_t* oo = reinterpret_cast<const uint16_t*>(a.out) + hr * D + g4 * 8;
+#pragma unroll
+    for (int j = 0; j < KSN; ++j) gf[j] = ldg16(go + j * 32);
+#pragma unroll
+    for (int j = 0; j < KS; ++j) qf[j] = j < KSN ? ldg16(q + j * 32) : ldg16(qr + (j - KSN) * 32);
+    uint16_t* qc = w.qcat + hr * DT + g4 * 8;
+    uint16_t* gc = w.gocat + hr * D + g4 * 8;
+#pragma unroll
+    for (int j = 0; j < KSN; ++j) {
+      const uint4 o = ldg16(oo + j * 32), gv = gf[j];
+      const uint32_t ow[4] = {o.x, o.y, o.z, o.w}, gw[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dl += to_f32<IO>((uint16_t)(ow[i] & 0xFFFFu)) * to_f32<IO>((uint16_t)(gw[i] & 0xFFFFu));
+        dl += to_f32<IO>((uint16_t)(ow[i] >> 16)) * to_f32<IO>((uint16_t)(gw[i] >> 16));
+      }
+      stg16(gc + j * 32, ntok > 0 ? gv : z4);
+    }
+#pragma unroll
+    for (int j = 0; j < KS; ++j) stg16(qc + j * 32, ntok > 0 ? qf[j] : z4);
+    dl += __shfl_xor(dl, 16);
+    dl += __shfl_xor(dl, 32);
+  }
+  const float m2 = a.sm_max[hr] * BLOG2E;
+  const float lsum = a.sm_sum[hr];
+  const float il = lsum > 0.f ? 1.f / lsum : 0.f;
+  const float sl2 = f.scale * BLOG2E;
+  if (zf) {   // the batch tokens the row selects; the others' dense entries are zeroed as the tiles go
+    for (int i = tid; i < (g.nk + 31) / 32; i += NW * 64) s_sel[i] = 0;
+    lds_barrier();
+    for (int i = tid; i < ntok; i += NW * 64) {
+      const int id = toks[i], tb = id - g.ks;
+      if ((uint32_t)id < (uint32_t)krows && tb >= 0 && tb < g.nk) atomicOr(&s_sel[tb >> 5], 1u << (tb & 31));
+    }
+  }
+  // zeros of this (row, head block)'s dense slice at the unselected tokens of [z0, z1): 16 threads per token,
+  // 16 bytes of one buffer each
+  auto zero_tokens = [&](int z0, int z1) __attribute__((always_inline)) {
+    const int q = tid & 15;
+    uint16_t* zb = (q < 8 ? w.dst : w.pt) + dbase + (q & 7) * 8;
+    for (int t = z0 + (tid >> 4); t < z1; t += NW * 4)
+      if (!((s_sel[t >> 5] >> (t & 31)) & 1u)) stg16(zb + (int64_t)t * g.kp, z4);
+  };
+
+  {
+    float agpr_hint = 0.f;   // dQ in AGPRs
+    asm volatile("" : "+a"(agpr_hint));
+  }
+  f32x4 dq[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  if (ntok > 0) {
+    struct Idx {
+      int nope, rope;       // lane: token lane % 8, lane / 8 of the wave's 8, clamped into range
+      uint32_t zero_rows;   // tokens whose id is out of range: they read row 0 and are zeroed once landed
+    };
+    auto tile_idx = [&](int t) __attribute__((always_inline)) {
+      const int tb = clamp_tile(t) * BT;
+      const int nvalid = ntok - tb < BT ? ntok - tb : BT;
+      const int32_t* ids = s_ids[t & 7];
+      const int first = ids[0];   // slots past the token list take the tile's first token (their P is 0)
+      const int k = wave * 8 + (lane & 7), k2 = wave * 8 + (lane >> 3);
+      int v = ids[k], u = ids[k2];
+      v = k < nvalid ? v : first;
+      u = k2 < nvalid ? u : first;
+      Idx ix;
+      const bool bad = (uint32_t)v >= (uint32_t)krows;
+      ix.zero_rows = (uint32_t)__builtin_amdgcn_ballot_w64(bad) & 0xFFu;
+      ix.nope = bad ? 0 : v;
+      ix.rope = (uint32_t)u >= (uint32_t)krows ? 0 : u;
+      return ix;
+    };
+    const uint32_t wsw = (uint32_t)(wave & 1) * 128;   // kv_swz of tokens 8 .. 15 against 0 .. 7: bit 3
+    const uint32_t rlane = (uint32_t)((lane & 7) ^ rswz(lane >> 3)) * 16;
+    auto gather_part = [&](int j, const Idx& ix, int buf) __attribute__((always_inline)) {
+      if (j < 8) {
+        uint32_t base = ((uint32_t)__builtin_amdgcn_readlane(ix.nope, j) * (D * 2) + kv_swz(j) * 16) ^ wsw;
+        asm volatile("" : "+s"(base));
+        lds_dma16_sbase_untracked(kb, base ^ (uint32_t)(lane * 16), nope_buf[buf] + (wave * 8 + j) * (D * 2));
+      } else {
+        uint32_t off = (uint32_t)ix.rope * (BDR * 2) + rlane;
+        asm volatile("" : "+v"(off));
+        lds_dma16_sbase_untracked(krb, off, rope_buf[buf] + wave * 1024);
+      }
+    };
+    // LDS addresses in buffer 0, the lane-dependent part (16-byte chunks permuted): S^T / dP^T operand (token
+    // 16 half + lane % 16, chunk 4 ks + lane / 16), ks = 4 a + b: ka[b] + 256 a + 16 rows half; rope kr[.] + 2048
+    // half. dQ operand (columns 16 blk .. + 16, tokens 4 (lane / 16) .. + 4 and 16 on), blk = 8 a + b: tv[b] +
+    // 256 a; rope tr[.]
+    uint32_t ka[4], kr[2], tv[8], trp[4];
+    {
+      const uint32_t nb0 = lds_addr(&nope_buf[0][0]), rb0 = lds_addr(&rope_buf[0][0]);
+      const int tok = g4 * 4 + (l16 >> 2), low = (l16 & 3) >> 1, sub = (l16 & 1) * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ka[i] = nb0 + l16 * (D * 2) + (((4 * i + g4) ^ kv_swz(l16)) * 16);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) kr[i] = rb0 + l16 * (BDR * 2) + (((4 * i + g4) ^ rswz(l16)) * 16);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) tv[i] = nb0 + tok * (D * 2) + (((2 * i + low) ^ kv_swz(tok)) * 16) + sub;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) trp[i] = rb0 + tok * (BDR * 2) + (((2 * i + low) ^ rswz(tok)) * 16) + sub;
+    }
+    uint16_t* const sp = &stage[wave][0][0];
+    uint16_t* const sd = &stage[wave][1][0];
+
+    wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    lds_barrier();   // every wave's ids landed (and s_sel cleared)
+    uint32_t zr0, zr1;   // zero_rows of the tile to compute next and of the one after it
+    {
+      const Idx i0 = tile_idx(0), i1 = tile_idx(1);
+      zr0 = i0.zero_rows;
+      zr1 = i1.zero_rows;
+#pragma unroll
+      for (int j = 0; j < GPW - 1; ++j) gather_part(j, i0, 0);
+#pragma unroll
+      for (int j = 0; j < GPW - 1; ++j) gather_part(j, i1, 1);
+    }
+    const int zper = ((g.nk + ntiles - 1) / ntiles + 15) / 16 * 16;   // dense tokens cleared per tile
+    uint4 db = z4;   // dS^T of the last tile: the dQ B operand
+    uint4 vb[VR];
+#pragma unroll
+    for (int j = 0; j < VR; ++j) vb[j] = z4;
+    // dQ operand of column block blk: address sets of the tile in use
+    uint32_t tvt[8], trt[4];
+    auto t_base = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) tvt[i] = tv[i] + (uint32_t)u * NOPE;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) trt[i] = trp[i] + (uint32_t)u * ROPE;
+    };
+    auto t_frag = [&](int blk) __attribute__((always_inline)) -> uint4 {
+      const uint32_t p = blk < D / 16 ? tvt[blk & 7] + (blk >> 3) * 256 : trt[blk - D / 16];
+      const uint2 lo = ds_read_tr_at(p);
+      const uint2 hi = ds_read_tr_at(p + (blk < D / 16 ? 16 * (D * 2) : 16 * (BDR * 2)));
+      return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
+    // ---- P and dS of tile u to the dense buffers, and the tile's share of the zeros: lane = token 16 half +
+    // lane % 16, heads 4 (lane / 16) .. + 4. Issued early in the next tile.
+    uint2 pv[2], dv[2];
+    int sid[2];
+    auto dense_load = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const uint32_t so = (uint32_t)((g4 * 4 + (l16 >> 2)) * SP + half * 16 + 4 * (l16 & 3)) * 2;
+        pv[half] = ds_read_tr(reinterpret_cast<uint8_t*>(sp) + so);
+        dv[half] = ds_read_tr(reinterpret_cast<uint8_t*>(sd) + so);
+        sid[half] = s_ids[u & 7][half * 16 + l16];
+      }
+    };
+    auto dense_store = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int tb = sid[half] - g.ks;   // token index within the batch
+        if (dense_ok && u * BT + half * 16 + l16 < ntok && (uint32_t)sid[half] < (uint32_t)krows && tb >= 0 &&
+            tb < g.nk) {
+          const int64_t di = dbase + (int64_t)tb * g.kp + wave * 16 + g4 * 4;
+          *reinterpret_cast<uint2*>(w.pt + di) = pv[half];
+          *reinterpret_cast<uint2*>(w.dst + di) = dv[half];
+        }
+      }
+      if (zf) zero_tokens(u * zper, min((u + 1) * zper, g.nk));
+    };
+    t_base(0);   // (tile 0's dQ step multiplies tile 0's rows by a zero dS)
+    int buf = 0;
+    for (int t = 0; t < ntiles; ++t) {
+      // this wave's gathers of tile t. The GPW loads of the tile after it were issued later, so at most GPW
+      // operations left means that these have landed; stores retire out of order with loads, so none
+      // is counted on (a wait that counted them read rows that had not landed). Two tiles ahead, the
+      // wait leaves room for the last tile's stores; one tile ahead it waited for them (743 us the call).
+      if (t == 0) wait_vmcnt<GPW - 1>(); else wait_vmcnt<GPW>();
+      if (zr0) {   // rare: rows out of range read as zeros
+        wait_vmcnt<0>();
+        for (int j = 0; j < 8; ++j)
+          if ((zr0 >> j) & 1u) {
+            *reinterpret_cast<uint4*>(nope_buf[buf] + (wave * 8 + j) * (D * 2) + lane * 16) = z4;
+            if (lane < 8) *reinterpret_cast<uint4*>(rope_buf[buf] + (wave * 8 + j) * (BDR * 2) + lane * 16) = z4;
+          }
+      }
+      lds_barrier();   // tile t resident; every wave is done with tile t - 2, whose buffer tile t + 2 takes
+      const Idx ix = tile_idx(t + 2);
+      zr0 = zr1;
+      zr1 = ix.zero_rows;
+      const int gbuf = __builtin_amdgcn_readfirstlane(buf ^ 2);
+      const uint32_t noff = (uint32_t)buf * NOPE, roff = (uint32_t)buf * ROPE;
+      uint32_t kat[4], krt[2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kat[i] = ka[i] + noff;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) krt[i] = kr[i] + roff;
+      auto k_frag = [&](int half, int ks) __attribute__((always_inline)) -> uint4 {
+        return lds_read16_at(ks < KSN ? kat[ks & 3] + (ks >> 2) * 256 + half * 16 * (D * 2)
+                                      : krt[ks - KSN] + half * 16 * (BDR * 2));
+      };
+      // ---- S^T and dP^T of both halves, the rope steps last; the loads of tile t + 2 on the chain
+      constexpr int KPF = 6;
+      f32x4 sv[2], dp[2];
+      uint4 af[KPF];
+#pragma unroll
+      for (int j = 0; j < KPF; ++j) af[j] = k_frag(j / KS, j % KS);
+      if (t > 0) dense_load(t - 1);
+      static_for<0, 2 * KS>([&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value, half = j / KS, ks = j % KS;
+        if constexpr (ks == 0) mfma16x2_vacc_first<IO>(sv[half], dp[half], af[j % KPF], qf[ks], gf[ks]);
+        else if constexpr (ks < KSN - 1) mfma16x2_vacc<IO, false>(sv[half], dp[half], af[j % KPF], qf[ks], gf[ks]);
+        else if constexpr (ks == KSN - 1) mfma16x2_vacc<IO, true>(sv[half], dp[half], af[j % KPF], qf[ks], gf[ks]);
+        else if constexpr (ks == KS - 1) {
+          mfma16_vacc_last2<IO>(sv[half], af[(j - 1) % KPF], qf[ks - 1], af[j % KPF], qf[ks]);
+          if constexpr (j - 1 + KPF < 2 * KS) af[(j - 1) % KPF] = k_frag((j - 1 + KPF) / KS, (j - 1 + KPF) % KS);
+        }
+        if constexpr (ks != KS - 2 && j + KPF < 2 * KS) af[j % KPF] = k_frag((j + KPF) / KS, (j + KPF) % KS);
+        if constexpr (j + VR >= 2 * KS) vb[j + VR - 2 * KS] = t_frag(j + VR - 2 * KS);   // dQ of tile t - 1
+        constexpr int gp = (j * GPW + 2 * KS - 1) / (2 * KS);   // the load scheduled at this step, if any
+        if constexpr (gp < GPW && gp * 2 * KS / GPW == j) {
+          if constexpr (gp < GPW - 1) gather_part(gp, ix, gbuf);
+          else ids_dma(t + 5);   // its slot held the ids of tile t - 3
+        }
+        if constexpr (j == 5)
+          if (t > 0) dense_store(t - 1);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      // ---- dQ^T += K^T dS^T of tile t - 1, with P and dS of tile t (fp32 -> io dtype) among its MFMAs:
+      // step i covers token i % 4 of the lane's four of half i / 4
+      const int nv = ntok - t * BT < BT ? ntok - t * BT : BT;
+      uint32_t pw[4], dw[4];
+      float pe = 0.f, de = 0.f;
+      auto p_step = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, half = i / 4;
+        const bool ok = half * 16 + g4 * 4 + i % 4 < nv;
+        const float x = __builtin_amdgcn_exp2f(sv[half][i % 4] * sl2 - m2) * il;
+        const float p = ok ? x : 0.f, ds = ok ? x * (dp[half][i % 4] - dl) * f.scale : 0.f;
+        if constexpr (i % 2 == 0) {
+          pe = p;
+          de = ds;
+        } else {
+          pw[i / 2] = pack2<IO>(pe, p);
+          dw[i / 2] = pack2<IO>(de, ds);
+        }
+        if constexpr (i % 4 == 3) {
+          const int so = l16 * SP + half * 16 + g4 * 4;
+          *reinterpret_cast<uint2*>(sp + so) = make_uint2(pw[2 * half], pw[2 * half + 1]);
+          *reinterpret_cast<uint2*>(sd + so) = make_uint2(dw[2 * half], dw[2 * half + 1]);
+        }
+      };
+      static_for<0, NB>([&](auto bc) __attribute__((always_inline)) {
+        constexpr int blk = decltype(bc)::value;
+        dq[blk] = Mfma<IO>::m16(vb[blk % VR], db, dq[blk]);
+        if constexpr (blk + VR < NB) vb[blk % VR] = t_frag(blk + VR);
+        if constexpr (blk % 3 == 1 && blk / 3 < 8) p_step(std::integral_constant<int, blk / 3>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      db = make_uint4(dw[0], dw[1], dw[2], dw[3]);
+      t_base(buf);   // the next iteration's dQ reads this tile
+      buf = (buf + 1) & 3;
+    }
+    dense_load(ntiles - 1);
+    dense_store(ntiles - 1);
+    // ---- dQ of the last tile (its rows are resident; t_base points at them)
+#pragma unroll
+    for (int j = 0; j < VR; ++j) vb[j] = t_frag(j);
+    static_for<0, NB>([&](auto bc) __attribute__((always_inline)) {
+      constexpr int blk = decltype(bc)::value;
+      dq[blk] = Mfma<IO>::m16(vb[blk % VR], db, dq[blk]);
+      if constexpr (blk + VR < NB) vb[blk % VR] = t_frag(blk + VR);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    wait_vmcnt<0>();   // the ring's last (unused) gathers land before the LDS is released
+  }
+
+  // ---- d_query | d_query_rope (zeros for rows without tokens): lane = its head, columns 16 blk + 4 (lane / 16) .. + 4
+  {
+    uint16_t* dqo = reinterpret_cast<uint16_t*>(a.dq) + hr * D + g4 * 4;
+    uint16_t* dqr = reinterpret_cast<uint16_t*>(a.dqr) + hr * BDR + g4 * 4;
+#pragma unroll
+    for (int blk = 0; blk < NB; ++blk) {
+      uint16_t* o = blk < D / 16 ? dqo + blk * 16 : dqr + (blk - D / 16) * 16;
+      *reinterpret_cast<uint2*>(o) =
+          make_uint2(pack2<IO>(dq[blk][0], dq[blk][1]), pack2<IO>(dq[blk][2], dq[blk][3]));
+    }
+  }
+  if (zf && ntok == 0) zero_tokens(0, g.nk);   // (s_sel was cleared behind a barrier)
+}
+
 // ---- staged library-GEMM rows to the outputs: key row kr of batch b (the last batch
 // with key_start[b] <= kr), t = kr - key_start[b], takes staged row boffk[b] + t when
 // t < nk and the batch has query rows; every other key row is zero. One thread per 8
@@ -589,6 +963,17 @@ template <int IO, int D>
 hipError_t launch_rows_d(const SfaBwdArgs& a, const SfaTokenLists& tl, const BwdWs& w, hipStream_t s) {
   const SfaArgs& f = a.f;
   if (f.total_rows > 0) {
+    if constexpr (D == r64::D) {
+      // whole blocks of 64 heads, gathers by 32-bit row offsets, the dense slices cleared by the kernel; and
+      // more than one round of the 32-head form's work-groups (below it, its eight waves a tile are the
+      // shorter latency: 70 rows 64 us against 70)
+      if (f.n1 % r64::NH == 0 && (int64_t)f.total_rows * (f.n1 / BH) > 256 && (uint64_t)f.key_rows * D * 2 <= (1ull << 32) && w.zfuse &&
+          w.max_nk <= 32 * r64::ZBW) {
+        hipLaunchKernelGGL(sfa_bwd_rows64_kernel<IO>, dim3(f.total_rows, f.n1 / r64::NH), dim3(r64::NW * 64), 0, s, a,
+                           tl, w);
+        return hipGetLastError();
+      }
+    }
     const dim3 grid(f.total_rows, (f.n1 + BH - 1) / BH);
     hipLaunchKernelGGL((sfa_bwd_rows_kernel<IO, D>), grid, dim3(BWV * 64), 0, s, a, tl, w);
   }
@@ -631,11 +1016,10 @@ hipError_t launch_place(const SfaBwdArgs& a, const BwdWs& w, hipStream_t s) {
 // ---- library GEMMs. hipBLASLt is loaded (dlopen) by the first backward call, so the
 // indexer / forward library has no load-time dependency on it. One handle per device,
 // created on that device's first backward call outside stream capture (the library
-// allocates its own small state then). The algorithm of a product is fixed per shape: the
-// entry of hipBLASLt's ranked heuristic list that a committed table names for the shape
-// (measured on this image's hipBLASLt), else the list's first entry. The list is a
-// deterministic function of the library build and the product's shape, so every process
-// uses the same kernel and gets the same bits; nothing is timed and the host never waits.
+// allocates its own small state then). The algorithm of a product is the first entry of
+// hipBLASLt's ranked heuristic list. The list is a deterministic function of the library
+// build and the product's shape, so every process uses the same kernel and gets the same
+// bits; nothing is timed and the host never waits.
 struct LtApi {
   decltype(&hipblasLtCreate) create = nullptr;
   decltype(&hipblasLtMatmulDescCreate) desc_create = nullptr;
@@ -689,20 +1073,6 @@ const LtApi& lt_api() {
   });
   return api;
 }
-
-// Committed algorithm choices: the position in the heuristic's ranked list for a product
-// shape (element size, output columns, key rows, contraction, dense row stride, split).
-// Measured at the reference's grad perf shape (perf_sfa_grad_triton.py:23) on this image's
-// hipBLASLt: the [d_key | d_key_rope] product runs 0.167 ms with entry 38 against 0.198 ms
-// with the first entry; for the d_value product the first entry is within 1% of the best.
-struct LtPick {
-  int esize, n_cols, nk, k;
-  int64_t kp;
-  int split, index;
-};
-constexpr LtPick LT_PICKS[] = {
-    {2, 576, 4096, 32768, 32768, 4, 38},
-};
 
 struct LtCache {
   std::mutex mu;
@@ -799,13 +1169,7 @@ hipError_t lt_gemm(hipDataType dt, int n_cols, int nk, int k, int split, const v
       if (api.heuristic(h, desc, la, lb, lc, lc, pref, LT_CANDIDATES, res, &nres) != HIPBLAS_STATUS_SUCCESS ||
           nres < 1)
         break;
-      int pick = 0;
-      const int esize = 2;   // bf16 / fp16 operands
-      for (const LtPick& p : LT_PICKS)
-        if (p.esize == esize && p.n_cols == n_cols && p.nk == nk && p.k == k && p.kp == kp && p.split == split &&
-            p.index < nres && res[p.index].workspaceSize <= LT_WS)
-          pick = p.index;
-      algo = res[pick].algo;
+      algo = res[0].algo;
       std::lock_guard<std::mutex> g(c.mu);
       c.algo[key] = algo;
     }
@@ -908,6 +1272,7 @@ hipError_t launch_sfa_bwd(const SfaBwdArgs& a, hipStream_t s) {
   }
   const int zbw = f.d == 128 ? dsa::BCfg<128>::ZBW : (f.d == 256 ? dsa::BCfg<256>::ZBW : dsa::BCfg<512>::ZBW);
   w.zfuse = f.n1 % 8 == 0 && (int64_t)max_nk <= 32 * (int64_t)zbw;
+  w.max_nk = max_nk;
 
   hipLaunchKernelGGL(dsa::sfa_bwd_geo_kernel, dim3(1), dim3(256), 0, s, f, w);
   if (!w.zfuse) {

@@ -1477,10 +1477,7 @@ __global__ __launch_bounds__(NWV * 64) void sfa_attn_kernel(SfaArgs a, int cap, 
 // form this replaces took 3,600 per single tile.
 //  * The ring holds two 32-token tiles (two work-groups' rings fill the LDS): the gathers of tile t+1
 //    ride on the S^T chain of tile t and have its softmax and PV to land. One barrier per tile.
-//  * Rows are unpadded (1024 B) and 16-byte chunk c of token t sits at c ^ swz(t), a bijection of
-//    t % 16 chosen for both readers: the 8 consecutive tokens of an S^T operand read differ in its low
-//    three bits, and the four tokens of a transposed V read in bits 2 and 3, so their 64-byte runs
-//    cover all 64 banks.
+//  * Rows are unpadded (1024 B), their chunks permuted by kv_swz.
 //  * A tile's scores come in two halves of 16 tokens (16x16x32 MFMAs, two head tiles sharing each K
 //    operand): the softmax of the first half runs under the S^T MFMAs of the second, that of the second
 //    under the PV MFMAs of the first. The last NPRE PV MFMAs of a tile run after the next barrier, under
@@ -1491,20 +1488,7 @@ constexpr int NW = 2;                             // waves, 32 heads each
 constexpr int KS = (D + DR) / 32, KSN = D / 32;   // S^T k-steps (18), of which nope (16)
 constexpr int NOPE = BN * D * 2;                  // bytes of a tile's nope rows
 constexpr int ROPE = BN * DR * 2;
-__host__ __device__ constexpr int swz(int t) {
-  return ((((t >> 1) ^ (t >> 3)) & 1) << 3) | ((t & 1) << 2) | (t & 2) | ((t >> 2) & 1);
-}
 }  // namespace w2
-
-// f(integral_constant I), f(I + 1), .. f(N - 1): an unrolled loop whose body may be of any size (the
-// compiler gives up on `#pragma unroll` of very large ones and moves the arrays they index to scratch)
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 template <int IO>
 __global__ __launch_bounds__(w2::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -1618,7 +1602,7 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
     if (j < RPW) {
       // row base, chunk permutation and lane in one VALU op (disjoint bits); the empty asm keeps
       // the address arithmetic at this point of the chain
-      uint32_t base = (uint32_t)__builtin_amdgcn_readlane(ix.nope, j) * (D * 2) + w2::swz(j & 15) * 16;
+      uint32_t base = (uint32_t)__builtin_amdgcn_readlane(ix.nope, j) * (D * 2) + kv_swz(j & 15) * 16;
       asm volatile("" : "+s"(base));
       lds_dma16_sbase_untracked(kb, base ^ (uint32_t)(lane * 16), nope_buf[buf] + (wave * RPW + j) * (D * 2));
     } else {
@@ -1681,20 +1665,18 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
     const int tok = kg * 8 + (l16 >> 2), low = (g4 & 1) * 2 + ((l16 & 3) >> 1);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      ka[b] = nb0 + l16 * (D * 2) + (((4 * b + g4) ^ w2::swz(l16)) * 16);
-      vlo[b] = nb0 + tok * (D * 2) + (((4 * b + low) ^ w2::swz(tok)) * 16) + (l16 & 1) * 8;
-      vhi[b] = nb0 + (tok + 4) * (D * 2) + (((4 * b + low) ^ w2::swz(tok + 4)) * 16) + (l16 & 1) * 8;
+      ka[b] = nb0 + l16 * (D * 2) + (((4 * b + g4) ^ kv_swz(l16)) * 16);
+      vlo[b] = nb0 + tok * (D * 2) + (((4 * b + low) ^ kv_swz(tok)) * 16) + (l16 & 1) * 8;
+      vhi[b] = nb0 + (tok + 4) * (D * 2) + (((4 * b + low) ^ kv_swz(tok + 4)) * 16) + (l16 & 1) * 8;
       asm volatile("" : "+v"(ka[b]), "+v"(vlo[b]), "+v"(vhi[b]));
     }
   }
   uint32_t kr = lds_addr(&rope_buf[0][0]) + (l16 >> 3) * 1024 + (g4 * 8 + (l16 & 7)) * 16;
   asm volatile("" : "+v"(kr));
-  typedef __attribute__((address_space(3), aligned(16))) u32x4v lds_u32x4;
   auto k_frag = [&](int half, int ks, int buf) __attribute__((always_inline)) -> uint4 {
     const uint32_t p = ks < KSN ? ka[ks & 3] + (ks >> 2) * 256 + half * 16 * (D * 2) + buf * w2::NOPE
                                 : kr + (ks - KSN) * 512 + half * 2048 + buf * w2::ROPE;
-    const u32x4v v = *(const lds_u32x4*)(uintptr_t)p;
-    return __builtin_bit_cast(uint4, v);
+    return lds_read16_at(p);
   };
   constexpr int NPV = 2 * ON;   // PV MFMAs per tile
   auto v_frag = [&](int m, int buf) __attribute__((always_inline)) -> uint4 {

@@ -238,8 +238,8 @@ int dsa_sfa_fwd_noalloc(const void* query, const void* query_rope, const void* k
  * area of 4 fp32 partials of sum_b min(act_k[b], s2) rows of [d_key | d_key_rope |
  * d_value],
  * a [total_rows * N1, D + 64] copy of [query | query_rope], 128 MiB for the library
- * GEMMs, and two dense io-dtype buffers of sum_b min(act_k[b], s2) * ceil64(rows_b *
- * N1) elements (rows_b = host_row_start[b+1] - host_row_start[b]). host_row_start [batch + 1] and
+ * GEMMs, and two dense io-dtype buffers of sum_b min(act_k[b], s2) * (ceil64(rows_b *
+ * N1), plus 64 where that is a multiple of 1024) elements (rows_b = host_row_start[b+1] - host_row_start[b]). host_row_start [batch + 1] and
  * host_act_k [batch] are host copies of the row offsets and kv lengths. Needs no
  * initialisation. No counterpart in the reference (it allocates its buffers per
  * call, sparse_flash_attention_grad_triton.py:634-642).
