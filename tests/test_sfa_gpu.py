@@ -535,3 +535,23 @@ def test_two_wave_form_climbing_scores(dev, dtype):
     torch.cuda.synchronize()
     assert torch.equal(out[:, :4], out[:, -4:]) and torch.equal(out[:, :4], out[:, 140:144])
     compare(out[:, :4], smax[:, :, :4], ssum[:, :, :4], *o, what=f"two-wave climbing {dtype}")
+
+
+@pytest.mark.parametrize("B", [24, 100, 129, 255])
+def test_decode_batches_that_do_not_divide_the_cus(dev, B):
+    """Decode batches whose splits are rounded down to one round of work-groups (24: 4 splits of 512
+    tokens, 100: 2; above 128 rows unsplit, through the token-list launch), short rows among them."""
+    N1, D, S2, count = 16, 512, 520, 512
+    q, k, _, qr, kr = _inputs(B, 1, S2, N1, D, "bf16", seed=31)
+    lens = [1 + (37 * b) % S2 for b in range(B)]
+    rng = np.random.RandomState(32)
+    si = np.full((B, 1, 1, count), -1, np.int32)
+    for b in range(B):
+        n = min(count, lens[b])
+        si[b, 0, 0, :n] = rng.permutation(lens[b])[:n]
+    kw = dict(scale_value=0.04, actual_seq_lengths_kv=lens, sparse_mode=3, return_softmax_lse=True)
+    out, smax, ssum = sparse_flash_attention(q.to(dev), k.to(dev), k.to(dev), torch.from_numpy(si).to(dev),
+                                             query_rope=qr.to(dev), key_rope=kr.to(dev), **kw)
+    torch.cuda.synchronize()
+    o = SFA.sparse_flash_attention(_np(q), _np(k), None, si, query_rope=_np(qr), key_rope=_np(kr), io_dtype="bf16", **kw)
+    compare(out, smax, ssum, *o, what=f"decode B={B}")
