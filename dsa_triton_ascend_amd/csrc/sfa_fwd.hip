@@ -2278,8 +2278,165 @@ hipError_t launch_attn_d(const SfaArgs& a, hipStream_t s, int cap, int splits, i
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- teacher sums, up to 64 heads (D = 512)
+// sfa_attn_kernel's TEACH for N1 <= 64: t_p[slot] = (1 / N1) sum_h exp(S scale - t_max[h]) / (t_sum[h] + 1e-8).
+// One work-group of four waves per query row, two work-groups a CU (two waves per SIMD): wave w takes head
+// block w % 2 and the 16-token half w / 2 of every 32-token tile, so no partial score leaves a wave.
+// S[head, token] on 16x16x32 MFMAs, heads as M (a lane holds 8 heads of one token: the head sum is in-lane,
+// then over the four lane groups), two head tiles sharing each K operand; Q^T with its rope in VGPRs. The
+// ring of two tiles is that of sfa_attn2_kernel. 512 rows of 2048 slots, 64 heads: 162 -> 98 us;
+// the form it replaces split each chain over wave pairs with an exchange and a barrier more a tile.
+template <int IO>
+__global__ __launch_bounds__(256, 2) void sfa_teach64_kernel(SfaArgs a, Ws ws) {
+  using w2::D;
+  constexpr int KS = w2::KS, KSN = w2::KSN, NW = 4, RPW = BN / NW, GPW = RPW + 2;
+  __shared__ __attribute__((aligned(1024))) uint8_t nope_buf[2][w2::NOPE];
+  __shared__ __attribute__((aligned(1024))) uint8_t rope_buf[2][w2::ROPE];
+  __shared__ __attribute__((aligned(16))) int32_t s_ids[4][BN];   // token-id ring (tiles t+1 .. t+3)
+  __shared__ float t_tp[2][2][BN];   // head-block sums of a tile's tokens, by tile parity
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hb = wave & 1, half = wave >> 1;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int r = a.total_rows - 1 - (int)blockIdx.x;   // long (late causal) rows first
+  const int n1 = a.n1;
+  const int ntok = __builtin_amdgcn_readfirstlane(ws.counts[r]);
+  if (ntok == 0) return;
+  const int32_t* toks = ws.tokens + (int64_t)r * ws.tstride;
+  const uint16_t* kb = reinterpret_cast<const uint16_t*>(a.k);
+  const uint16_t* krb = reinterpret_cast<const uint16_t*>(a.kr);
+  const int ntiles = (ntok + BN - 1) / BN;
+  auto clamp_tile = [&](int t) { return t < ntiles ? t : ntiles - 1; };
+  auto ids_dma = [&](int t) {
+    if (lane < 2)
+      lds_dma16_sbase_untracked(toks, (uint32_t)(clamp_tile(t) * BN + wave * 8) * 4 + lane * 16,
+                                &s_ids[0][0] + __builtin_amdgcn_readfirstlane((t & 3) * BN + wave * 8));
+  };
+#pragma unroll
+  for (int t = 0; t < 3; ++t) ids_dma(t);
+  // Q fragments: head 32 hb + 16 n + lane % 16, 8 elements at 32 ks + 8 (lane / 16); padded heads are zero
+  uint4 qf[KS][2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const int h = hb * 32 + 16 * n + l16;
+    const int64_t hr = (int64_t)r * n1 + min(h, n1 - 1);
+    const uint16_t* q = reinterpret_cast<const uint16_t*>(a.q) + hr * D + g4 * 8;
+    const uint16_t* qr = reinterpret_cast<const uint16_t*>(a.qr) + hr * DR + g4 * 8;
+#pragma unroll
+    for (int j = 0; j < KS; ++j) qf[j][n] = ldg16_or0(h < n1, j < KSN ? q + j * 32 : qr + (j - KSN) * 32);
+  }
+  // statistics of the heads the lane's scores belong to: 32 hb + 16 n + 4 (lane / 16) + i
+  float tm[2][4], ti[2][4];
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int h = hb * 32 + 16 * n + g4 * 4 + i;
+      const int64_t hr = (int64_t)r * n1 + min(h, n1 - 1);
+      tm[n][i] = h < n1 ? a.t_max[hr] * LOG2E : 0.f;
+      ti[n][i] = h < n1 ? 1.f / (a.t_sum[hr] + 1e-8f) : 0.f;   // padded heads contribute 0
+    }
+  const float sl2 = a.scale * LOG2E, inv_n1 = 1.f / n1;
+  float* const tp = a.t_p + (int64_t)r * a.t_ld;
+
+  // (slot ids are clipped into the key tensor by the slot-list kernel)
+  const uint32_t wsw = (uint32_t)(wave & 1) * 128;   // kv_swz of tokens 8 .. 15 against 0 .. 7: bit 3
+  struct Idx { int nope, rope; };
+  auto tile_idx = [&](int t) __attribute__((always_inline)) {
+    const int tb = clamp_tile(t) * BN;
+    const int nvalid = ntok - tb < BN ? ntok - tb : BN;
+    const int32_t* ids = s_ids[t & 3];
+    const int first = ids[0];   // slots past the list take the tile's first
+    const int k = wave * 8 + (lane & 7);
+    Idx ix;
+    ix.nope = k < nvalid ? ids[k] : first;
+    ix.rope = ix.nope;   // lane -> token lane % 8, chunk lane / 8 (rope_off's order)
+    return ix;
+  };
+  auto gather_part = [&](int j, const Idx& ix, int buf) __attribute__((always_inline)) {
+    if (j < RPW) {
+      uint32_t base = ((uint32_t)__builtin_amdgcn_readlane(ix.nope, j) * (D * 2) + kv_swz(j) * 16) ^ wsw;
+      asm volatile("" : "+s"(base));
+      lds_dma16_sbase_untracked(kb, base ^ (uint32_t)(lane * 16), nope_buf[buf] + (wave * 8 + j) * (D * 2));
+    } else {
+      uint32_t off = (uint32_t)ix.rope * (DR * 2) + (uint32_t)(lane >> 3) * 16;
+      asm volatile("" : "+v"(off));
+      lds_dma16_sbase_untracked(krb, off, rope_buf[buf] + wave * 1024);
+    }
+  };
+  // K operand of this wave's half: token 16 half + lane % 16, chunk 4 ks + lane / 16 (addresses as sfa_attn2_kernel)
+  uint32_t ka[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    ka[i] = lds_addr(&nope_buf[0][0]) + (half * 16 + l16) * (D * 2) + (((4 * i + g4) ^ kv_swz(l16)) * 16);
+  const uint32_t kr = lds_addr(&rope_buf[0][0]) + half * 2048 + (l16 >> 3) * 1024 + (g4 * 8 + (l16 & 7)) * 16;
+  // the sums of tile u over the head blocks (written before the last barrier) to t_p
+  auto teach_store = [&](int u) __attribute__((always_inline)) {
+    if (tid < BN && u * BN + tid < ntok) tp[u * BN + tid] = (t_tp[u & 1][0][tid] + t_tp[u & 1][1][tid]) * inv_n1;
+  };
+
+  wait_vmcnt<0>();
+  asm volatile("" ::: "memory");
+  lds_barrier();   // every wave's ids landed
+  {
+    const Idx ix = tile_idx(0);
+#pragma unroll
+    for (int j = 0; j < GPW - 1; ++j) gather_part(j, ix, 0);
+  }
+  for (int t = 0; t < ntiles; ++t) {
+    const int buf = t & 1;
+    if (t == 0) wait_vmcnt<0>(); else wait_vmcnt<1>();   // this wave's gathers of tile t (the ids copy follows them)
+    lds_barrier();   // tile t resident, tile t-1's sums visible; every wave is done with tile t-1's buffer
+    if (t > 0) teach_store(t - 1);
+    const Idx ix = tile_idx(t + 1);
+    const int gbuf = __builtin_amdgcn_readfirstlane(buf ^ 1);
+    uint32_t kat[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) kat[i] = ka[i] + (uint32_t)buf * w2::NOPE;
+    const uint32_t krt = kr + (uint32_t)buf * w2::ROPE;
+    auto k_frag = [&](int ks) __attribute__((always_inline)) -> uint4 {
+      return lds_read16_at(ks < KSN ? kat[ks & 3] + (ks >> 2) * 256 : krt + (ks - KSN) * 512);
+    };
+    constexpr int KPF = 4;
+    f32x4 c[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    uint4 af[KPF];
+#pragma unroll
+    for (int j = 0; j < KPF; ++j) af[j] = k_frag(j);
+    static_for<0, KS>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+#pragma unroll
+      for (int n = 0; n < 2; ++n) c[n] = Mfma<IO>::m16(qf[j][n], af[j % KPF], c[n]);
+      if constexpr (j + KPF < KS) af[j % KPF] = k_frag(j + KPF);
+      constexpr int gp = (j * GPW + KS - 1) / KS;   // the load scheduled at this step, if any
+      if constexpr (gp < GPW && gp * KS / GPW == j) {
+        if constexpr (gp < GPW - 1) gather_part(gp, ix, gbuf);
+        else ids_dma(t + 3);   // slot (t + 3) % 4 held the ids of tile t - 1
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    float e = 0.f;
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e += __builtin_amdgcn_exp2f(__builtin_fmaf(c[n][i], sl2, -tm[n][i])) * ti[n][i];
+    e = add_half_swap(e);   // the block's other head groups of the token
+    e += __shfl_xor(e, 16);
+    if (lane < 16) t_tp[buf][hb][half * 16 + l16] = e;
+  }
+  wait_vmcnt<0>();   // the last (unused) gathers land before the LDS is released
+  lds_barrier();
+  teach_store(ntiles - 1);
+}
+
 template <int IO, int D>
 hipError_t launch_teach_d(const SfaArgs& a, hipStream_t s, int cap, Ws ws) {
+  if constexpr (D == w2::D) {
+    if (a.n1 <= 64 && (uint64_t)a.key_rows * D * 2 <= (1ull << 32)) {   // 32-bit row offsets
+      hipLaunchKernelGGL(sfa_teach64_kernel<IO>, dim3(a.total_rows), dim3(256), 0, s, a, ws);
+      return hipGetLastError();
+    }
+  }
   if (a.n1 <= 64)
     hipLaunchKernelGGL((sfa_attn_kernel<IO, D, 64, true>), dim3(a.total_rows, 1), dim3(NWV * 64), 0, s, a, cap, 1, 0,
                        ws);

@@ -313,3 +313,28 @@ def test_grad_bitwise_reproducible_across_processes(tmp_path):
         files.append(np.load(f))
     for name in ("dq", "dk", "dv", "dqr", "dkr"):
         assert np.array_equal(files[0][name], files[1][name]), f"{name} differs between processes"
+
+
+@pytest.mark.parametrize("N1,dtype", [(64, "bf16"), (64, "fp16"), (128, "bf16")])
+def test_grad_64_head_rows(dev, N1, dtype):
+    """D = 512 with whole blocks of 64 heads and more rows than one round of the 32-head form (the
+    64-head rows kernel): rows of 1 .. 70 tokens (every remainder of the 32-token tile), two batches
+    of different lengths, rows past act_q and causally empty ones, against the oracle; and the same
+    bits from a workspace filled with NaN bytes (the kernel writes every zero the products read)."""
+    from dsa_triton_ascend_amd.sparse_flash_attention_grad import GradPlan, INT64_MAX
+    B, S1, S2, count, D, act_q, act_k = 2, 140, 150, 70, 512, [140, 100], [150, 90]
+    got, want = _run_case(dev, B, S1, S2, N1, count, 1, 3, D, dtype, act_q, act_k)
+    _check(got, want, dtype, S1, f"64-head rows N1={N1} {dtype}")
+    q, k, _, qr, kr, do = (x.to(dev) for x in _inputs(B, S1, S2, N1, D, dtype))
+    si = torch.from_numpy(_ref_indices(B, S1, S2, count, 1, 3, act_q, act_k)).to(dev)
+    scale = 1.0 / math.sqrt(D + 64)
+    out, smax, ssum = sparse_flash_attention(q, k, k, si, scale_value=scale, actual_seq_lengths_query=act_q,
+                                             actual_seq_lengths_kv=act_k, query_rope=qr, key_rope=kr, sparse_mode=3,
+                                             return_softmax_lse=True)
+    plan = GradPlan(q, k, k, si, do, out, smax, ssum, scale, qr, kr, act_q, act_k, 1, "BSND", 3, INT64_MAX, INT64_MAX,
+                    False)
+    plan.ws.fill_(0xFF)
+    again = plan.run()
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dq", "dk", "dv", "dqr", "dkr"), again, got):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"N1={N1}: {name} differs"

@@ -251,3 +251,10 @@ def test_kl_loss_fp32_weights(dev, dtype):
     """float32 weights (the same values as the io-dtype case): the key-major d_key_index pass
     then takes the hi / lo split of ds instead of the exact-weight form."""
     run(dev, 1, 4, 1024, 32, 512, 64, 128, 512, dtype, pattern="repeated", w_f32=True)
+
+
+@pytest.mark.parametrize("N1,dtype", [(64, "bf16"), (32, "fp16")])
+def test_kl_loss_teacher_rows_of_every_length(dev, N1, dtype):
+    """D = 512 with at most 64 heads (the 64-head teacher): 70 rows of 1 .. 70 slots, every remainder
+    of its 32-slot tiles and 16-slot halves, and a second batch of shorter lengths."""
+    run(dev, 2, 70, 70, N1, 512, 64, 128, 70, dtype, "causal_random", act_q=[70, 40], act_k=[70, 45], loose=True)
