@@ -36,6 +36,9 @@
 //         [head][token];
 //       * dQ[head, col] += dS K, each wave owning an eighth of the 32-column
 //         blocks, the K operand read with ds_read_b64_tr_b16 from the tile;
+//     or, at D = 512 with whole blocks of 64 heads and more rows than one round of
+//     those work-groups, sfa_bwd_rows64_kernel (four waves of 16 heads, nothing
+//     exchanged between waves; below);
 //  4. two library GEMMs per batch (hipBLASLt, loaded on first use; a fixed algorithm per
 //     shape, so results are reproducible across processes; bf16/fp16 in and out, fp32
 //     accumulation): [d_key | d_key_rope] = dS_T [q | q_rope] (one product: the rows

@@ -2407,6 +2407,7 @@ __global__ __launch_bounds__(256, 2) void sfa_teach64_kernel(SfaArgs a, Ws ws) {
       constexpr int j = decltype(jc)::value;
 #pragma unroll
       for (int n = 0; n < 2; ++n) c[n] = Mfma<IO>::m16(qf[j][n], af[j % KPF], c[n]);
+      __builtin_amdgcn_sched_barrier(0);   // the step's loads stay behind its MFMAs
       if constexpr (j + KPF < KS) af[j % KPF] = k_frag(j + KPF);
       constexpr int gp = (j * GPW + KS - 1) / KS;   // the load scheduled at this step, if any
       if constexpr (gp < GPW && gp * KS / GPW == j) {
