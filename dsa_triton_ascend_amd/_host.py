@@ -79,11 +79,15 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
 UPLOAD_MAX = 8192   # dsa_upload_i32's limit
 
 
-def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | None = None):
+def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | None = None, wait: bool = True):
     """The int32 length and offset arrays of a call on the device, views of one tensor (each padded
     to 16 bytes), written by one launch on the current stream (dsa_upload_i32); `zero` (a
     byte tensor) is cleared by the same launch. More values than a launch takes, or a device
-    that is not the current one, go by a copy."""
+    that is not the current one, go by a copy. With `wait` the host waits until the arrays and
+    all that the caller put on this stream before are in place: a kept plan may run on any
+    stream, and these arrays bound its addresses. A call that builds its plan and runs it at
+    once, on one stream, needs no wait. Under stream capture there is none to wait for: the
+    write is a node of the graph, and a plan built there runs in that graph."""
     flat, sizes = array("i"), []
     try:
         for a in arrays:
@@ -100,9 +104,11 @@ def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | N
         _lib.check(lib.dsa_upload_i32(flat.buffer_info()[0], n, t.data_ptr(), ptr(zero),
                                       0 if zero is None else zero.numel(), stream_ptr(device)), "dsa_upload_i32")
     else:
-        t = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=True)
         if zero is not None:
             zero.zero_()
+        t = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=True)
+    if wait and not torch.cuda.is_current_stream_capturing():
+        torch.cuda.current_stream(device).synchronize()
     return t.split(sizes)
 
 

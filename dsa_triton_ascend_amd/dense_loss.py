@@ -75,7 +75,7 @@ def dense_lightning_indexer_softmax_lse(query_index, key_index, weights, actual_
     wdt = H.dtype_code(weights.dtype, "weights", allow_f32=True)
     B, S1, Nidx1, Didx = query_index.shape
     S2 = key_index.shape[1]
-    act_q, act_k = H.upload(lib, dev, aq, ak)
+    act_q, act_k = H.upload(lib, dev, aq, ak, wait=False)
     qi, ki, w = query_index.contiguous(), key_index.contiguous(), weights.contiguous()
     mx = torch.empty((B, 1, S1), dtype=torch.float32, device=dev)
     sm = torch.empty((B, 1, S1), dtype=torch.float32, device=dev)
@@ -90,13 +90,13 @@ npu_dense_lightning_indexer_softmax_lse = dense_lightning_indexer_softmax_lse
 
 
 class DenseLossPlan:
-    """Validated arguments, outputs and workspace of one dense loss call; ``run()``
-    launches on the current stream."""
+    """Validated arguments, outputs and workspace of one dense loss call, all in place when
+    the constructor returns; ``run()`` launches on the current stream, which may be another one."""
 
     def __init__(self, query, key, query_index, key_index, weights, softmax_max, softmax_sum,
                  softmax_max_index=None, softmax_sum_index=None, scale_value=1.0, query_rope=None,
                  key_rope=None, actual_seq_qlen=None, actual_seq_klen=None, layout="BSND",
-                 sparse_mode=3, pre_tokens=INT64_MAX, next_tokens=INT64_MAX):
+                 sparse_mode=3, pre_tokens=INT64_MAX, next_tokens=INT64_MAX, *, _wait=True):
         # the reference's checks (:667-706)
         if query.dim() != 4 or key.dim() != 4:
             raise ValueError("query and key must be 4D BSND tensors")
@@ -165,7 +165,7 @@ class DenseLossPlan:
         self.loss = torch.empty(1, dtype=torch.float32, device=dev)
         self.ws_bytes = lib.dsa_dense_li_grad_workspace_bytes(B, S1, S2, Didx)
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.d_aq, self.d_ak = H.upload(lib, dev, aq, ak)
+        self.d_aq, self.d_ak = H.upload(lib, dev, aq, ak, wait=_wait)
         self.lib, self.dev = lib, dev
         self.io = H.dtype_code(query.dtype, "query")
         self.wdt = H.dtype_code(weights.dtype, "weights", allow_f32=True)
@@ -192,7 +192,8 @@ def dense_loss_backward(query, key, query_index, key_index, weights, softmax_max
     dense_loss_backward_triton.py:709-774)."""
     return DenseLossPlan(query, key, query_index, key_index, weights, softmax_max, softmax_sum,
                          softmax_max_index, softmax_sum_index, scale_value, query_rope, key_rope,
-                         actual_seq_qlen, actual_seq_klen, layout, sparse_mode, pre_tokens, next_tokens).run()
+                         actual_seq_qlen, actual_seq_klen, layout, sparse_mode, pre_tokens, next_tokens,
+                         _wait=False).run()
 
 
 def dense_lightning_indexer_grad_kl_loss(query, key, query_index, key_index, weights, softmax_max,

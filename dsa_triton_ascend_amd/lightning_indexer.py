@@ -30,11 +30,13 @@ class IndexerPlan:
     """Validated arguments of one lightning_indexer call: output buffers, the
     int32 index arrays the C ABI takes and the score scratch. ``score()`` and
     ``topk()`` launch the two kernels on the current stream (the bench times
-    them separately); ``run()`` does both."""
+    them separately); ``run()`` does both. All that the constructor sets up is in place when it
+    returns, so a plan may run on another stream than it was built on (calls of one plan share
+    its buffers and are ordered by the caller)."""
 
     def __init__(self, query, key, weights, actual_seq_lengths_query=None,
                  actual_seq_lengths_key=None, block_table=None, layout_query="BSND",
-                 layout_key="BSND", sparse_count=2048, sparse_mode=3, return_value=False):
+                 layout_key="BSND", sparse_count=2048, sparse_mode=3, return_value=False, *, _wait=True):
         is_pa = layout_key == "PA_BSND"
         if block_table is not None and not is_pa:
             raise ValueError("PA_BSND / block_table not supported in triton lightning_indexer")
@@ -109,7 +111,7 @@ class IndexerPlan:
         tw = int(self.lib.dsa_li_topk_workspace_bytes(total_rows, N2, S2, self.k))
         self.topk_ws = torch.empty(tw, dtype=torch.uint8, device=dev) if tw > 0 else None
         self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(self.lib, dev, row_start, key_start,
-                                                                            act_q, act_k)
+                                                                            act_q, act_k, wait=_wait)
         self.max_rows = max(row_start[b + 1] - row_start[b] for b in range(B)) if B else 0
         self.max_kv = max(act_k) if act_k else 0
 
@@ -170,7 +172,7 @@ def lightning_indexer(query, key, weights, actual_seq_lengths_query=None,
     any other layout with a block_table raises as the reference does."""
     return IndexerPlan(query, key, weights, actual_seq_lengths_query, actual_seq_lengths_key,
                        block_table, layout_query, layout_key, sparse_count, sparse_mode,
-                       return_value).run()
+                       return_value, _wait=False).run()
 
 
 class LightningIndexer(torch.nn.Module):

@@ -20,16 +20,16 @@ from .sparse_flash_attention import AttentionPlan
 class PrefillPlan:
     def __init__(self, index_query, index_key, index_weights, query, key, query_rope, key_rope,
                  cu_seqlens, sparse_count=2048, scale_value=1.0, sparse_mode=3,
-                 return_softmax_lse=False, return_value=False):
+                 return_softmax_lse=False, return_value=False, *, _wait=True):
         self.indexer = IndexerPlan(index_query, index_key, index_weights, cu_seqlens, cu_seqlens,
                                    layout_query="TND", layout_key="TND", sparse_count=sparse_count,
-                                   sparse_mode=sparse_mode, return_value=return_value)
+                                   sparse_mode=sparse_mode, return_value=return_value, _wait=False)
         self.attention = AttentionPlan(query, key, key, self.indexer.idx, scale_value,
                                        actual_seq_lengths_query=cu_seqlens,
                                        actual_seq_lengths_kv=cu_seqlens, query_rope=query_rope,
                                        key_rope=key_rope, sparse_block_size=1, layout_query="TND",
                                        layout_kv="TND", sparse_mode=sparse_mode,
-                                       return_softmax_lse=return_softmax_lse)
+                                       return_softmax_lse=return_softmax_lse, _wait=_wait)
         if self.attention.si.data_ptr() != self.indexer.idx.data_ptr():
             raise RuntimeError("attention plan does not read the indexer's index buffer in place")
 
@@ -52,4 +52,5 @@ def dsa_prefill(index_query, index_key, index_weights, query, key, query_rope, k
                 sparse_count=2048, scale_value=1.0, sparse_mode=3, return_softmax_lse=False):
     """One-shot form of ``PrefillPlan(...).run()``."""
     return PrefillPlan(index_query, index_key, index_weights, query, key, query_rope, key_rope,
-                       cu_seqlens, sparse_count, scale_value, sparse_mode, return_softmax_lse).run()
+                       cu_seqlens, sparse_count, scale_value, sparse_mode, return_softmax_lse,
+                       _wait=False).run()

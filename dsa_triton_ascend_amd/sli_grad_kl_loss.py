@@ -56,13 +56,13 @@ def _check_shapes(query, key, query_index, key_index, weights, sparse_indices, s
 
 
 class KLLossPlan:
-    """Validated arguments, outputs and workspace of one call; ``run()`` launches on
-    the current stream."""
+    """Validated arguments, outputs and workspace of one call, all in place when the
+    constructor returns; ``run()`` launches on the current stream, which may be another one."""
 
     def __init__(self, query, key, query_index, key_index, weights, sparse_indices, softmax_max,
                  softmax_sum, query_rope=None, key_rope=None, actual_seq_qlen=None,
                  actual_seq_klen=None, scale_value=1.0, layout="BSND", sparse_mode=3,
-                 pre_tokens=INT64_MAX, next_tokens=INT64_MAX, deterministic=False):
+                 pre_tokens=INT64_MAX, next_tokens=INT64_MAX, deterministic=False, *, _wait=True):
         # validation: the reference's conditions (:510-514)
         if layout != "BSND":
             raise ValueError("Only BSND layout is supported in triton path")
@@ -105,7 +105,7 @@ class KLLossPlan:
         self.loss = torch.empty(1, dtype=torch.float32, device=dev)
         self.ws_bytes = lib.dsa_sli_grad_workspace_bytes(B, S1, S2, topk, Didx)
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
-        self.d_aq, self.d_ak = H.upload(lib, dev, act_q, act_k)
+        self.d_aq, self.d_ak = H.upload(lib, dev, act_q, act_k, wait=_wait)
         self.lib, self.io, self.wdt, self.dev = lib, io, wdt, dev
         self.dims = (B, S1, S2, N1, D, Dr, Nidx1, Didx, topk)
         self.scale = float(scale_value)
@@ -131,7 +131,7 @@ def sparse_lightning_indexer_grad_kl_loss(query, key, query_index, key_index, we
     sparse_lightning_indexer_grad_kl_loss_triton.py:496-508)."""
     return KLLossPlan(query, key, query_index, key_index, weights, sparse_indices, softmax_max,
                       softmax_sum, query_rope, key_rope, actual_seq_qlen, actual_seq_klen, scale_value,
-                      layout, sparse_mode, pre_tokens, next_tokens, deterministic).run()
+                      layout, sparse_mode, pre_tokens, next_tokens, deterministic, _wait=False).run()
 
 
 class SparseLightningIndexerGradKLLoss(torch.nn.Module):

@@ -27,14 +27,15 @@ VALID_N1 = (1, 2, 4, 8, 16, 32, 64, 128)
 
 class AttentionPlan:
     """Validated arguments of one sparse_flash_attention call (outputs,
-    workspace, int32 index arrays); ``run()`` launches on the current stream."""
+    workspace, int32 index arrays), all in place when the constructor returns;
+    ``run()`` launches on the current stream, which may be another one."""
 
     def __init__(self, query, key, value, sparse_indices, scale_value=1.0, block_table=None,
                  actual_seq_lengths_query=None, actual_seq_lengths_kv=None,
                  query_rope=None, key_rope=None, sparse_block_size=1,
                  layout_query="BSND", layout_kv="BSND", sparse_mode=0,
                  pre_tokens=INT64_MAX, next_tokens=INT64_MAX, attention_mode=2,
-                 return_softmax_lse=False, block_size=0, kv_splits=0):
+                 return_softmax_lse=False, block_size=0, kv_splits=0, *, _wait=True):
         # validation: same conditions and messages as the reference (:1341-1351)
         if attention_mode != 2:
             raise ValueError("Only attention_mode=2 (MLA-absorb) is supported")
@@ -145,7 +146,7 @@ class AttentionPlan:
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
         zero = self.ws[:lib.dsa_sfa_workspace_zero_bytes()] if self.ws_bytes else None
         self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(lib, dev, row_start, key_start, act_q,
-                                                                            act_k, zero=zero)
+                                                                            act_k, zero=zero, wait=_wait)
         self.act_q, self.act_k, self.row_start = act_q, act_k, row_start
         self.key_rows = kk.numel() // D
 
@@ -179,7 +180,7 @@ def sparse_flash_attention(query, key, value, sparse_indices, scale_value=1.0, b
                          actual_seq_lengths_query, actual_seq_lengths_kv, query_rope, key_rope,
                          sparse_block_size, layout_query, layout_kv, sparse_mode, pre_tokens,
                          next_tokens, attention_mode, return_softmax_lse, block_size,
-                         kv_splits).run()
+                         kv_splits, _wait=False).run()
 
 
 class SparseFlashAttention(torch.nn.Module):

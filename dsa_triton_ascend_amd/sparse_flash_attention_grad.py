@@ -27,12 +27,13 @@ VALID_N1 = (1, 2, 4, 8, 16, 32, 64, 128)
 
 class GradPlan:
     """Validated arguments of one sparse_flash_attention_grad call (outputs, workspace,
-    int32 index arrays); ``run()`` launches on the current stream."""
+    int32 index arrays), all in place when the constructor returns; ``run()`` launches on the
+    current stream, which may be another one."""
 
     def __init__(self, query, key, value, sparse_indices, d_out, out, softmax_max, softmax_sum,
                  scale_value=1.0, query_rope=None, key_rope=None, actual_seq_lengths_query=None,
                  actual_seq_lengths_kv=None, sparse_block_size=1, layout="BSND", sparse_mode=3,
-                 pre_tokens=INT64_MAX, next_tokens=INT64_MAX, deterministic=False):
+                 pre_tokens=INT64_MAX, next_tokens=INT64_MAX, deterministic=False, *, _wait=True):
         # validation: same conditions and messages as the reference (:544-594)
         if pre_tokens != INT64_MAX or next_tokens != INT64_MAX:
             raise ValueError("pre_tokens/next_tokens only support default INT64_MAX")
@@ -135,7 +136,7 @@ class GradPlan:
             raise ValueError("dsa_sfa_bwd_workspace_bytes rejected the shapes")
         self.ws = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
         self.d_row_start, self.d_key_start, self.d_aq, self.d_ak = H.upload(lib, dev, row_start, key_start or [0],
-                                                                            act_q, act_k)
+                                                                            act_q, act_k, wait=_wait)
 
     def run(self):
         _lib.check(self.lib.dsa_sfa_bwd(
@@ -162,7 +163,7 @@ def sparse_flash_attention_grad(query, key, value, sparse_indices, d_out, out, s
     return GradPlan(query, key, value, sparse_indices, d_out, out, softmax_max, softmax_sum,
                     scale_value, query_rope, key_rope, actual_seq_lengths_query,
                     actual_seq_lengths_kv, sparse_block_size, layout, sparse_mode, pre_tokens,
-                    next_tokens, deterministic).run()
+                    next_tokens, deterministic, _wait=False).run()
 
 
 class SparseFlashAttentionGrad(torch.nn.Module):

@@ -330,6 +330,50 @@ def test_upload_i32_rejects_bad_arguments():
     assert lib.dsa_upload_i32(p, 0, None, None, 0, None) == _lib.DSA_OK   # nothing to do: no launch
 
 
+@pytest.mark.parametrize("n", [3, 9000])
+@pytest.mark.parametrize("wait", [True, False])
+def test_upload_wait_and_capture(monkeypatch, n, wait):
+    """A kept plan's arrays are in place when its constructor returns (its run() may be on another
+    stream): the wait follows the launch, or the copy that large arrays take, and the clearing.
+    Under stream capture the launch is recorded and nothing waits."""
+    from dsa_triton_ascend_amd import _host as H
+    done = []
+
+    class Lib:
+        def dsa_upload_i32(self, *a):
+            done.append("launch")
+            return 0
+
+    class Stream:
+        def synchronize(self):
+            done.append("wait")
+
+    class Zero:
+        def data_ptr(self):
+            return 64
+
+        def numel(self):
+            return 16
+
+        def zero_(self):
+            done.append("zero")
+
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(H, "stream_ptr", lambda device: 7)
+    values = list(range(n))
+    (got,) = H.upload(Lib(), torch.device("cpu"), values, zero=Zero(), wait=wait)
+    assert done == (["launch"] if n <= H.UPLOAD_MAX else ["zero"]) + ["wait"] * wait
+    if n > H.UPLOAD_MAX:
+        assert got[:n].tolist() == values
+    if n <= H.UPLOAD_MAX:
+        capturing[0], done[:] = True, []
+        H.upload(Lib(), torch.device("cpu"), values, wait=wait)
+        assert done == ["launch"]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("counts", [(1, 0, 3, 1), (14, 14, 14, 14), (57,), (960,), (961, 2), (8192,), (8193, 5)])
 def test_upload_of_length_arrays(counts):
