@@ -1691,9 +1691,7 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
   constexpr int KPF = 5;    // S^T operands in flight
   static_assert(NPRE <= VR && NPRE <= ON && GPW <= 2 * KS, "deferred PV; at most one load per step");
   uint4 vb[VR];
-  uint4 pb[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};   // P^T B operands of the tile's halves
-#pragma unroll
-  for (int m = 0; m < VR; ++m) vb[m] = make_uint4(0, 0, 0, 0);   // the first tile's deferred MFMAs add zeros
+  uint4 pb[2];   // P^T B operands of the tile's halves
   auto pv = [&](int m) __attribute__((always_inline)) { o[m % ON] = Mfma<IO>::m32(vb[m % VR], pb[m / ON], o[m % ON]); };
   float alpha = 1.f, sm_mb = 0.f, sm_mx = 0.f, sm_sum = 0.f;
   float sc[8];   // raw scores of a half: the lane's head, tokens 8 (lane / 32) + j
@@ -1701,6 +1699,9 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
   // that the lane holds 8 tokens of head lane % 32; 1 the max and the exponent reference; 2-5 two
   // exponentials each, into pb[half]
   constexpr int NST = 6;
+  auto max8 = [&]() __attribute__((always_inline)) {
+    return fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+  };
   auto smx = [&](int st, int half, int t, f32x4& c0, f32x4& c1) __attribute__((always_inline)) {
     if (st == 0) {
 #pragma unroll
@@ -1714,7 +1715,7 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) sc[j] = kg * 8 + j < nvalid ? sc[j] : -INFINITY;
     } else if (st == 1) {
-      sm_mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+      sm_mx = max8();
       // a half past the row's tokens leaves the reference alone (its max is -inf; a tile's first half holds a token)
       const float mx = max_half_swap(sm_mx) * cpos;
       m_true = fmaxf(m_true, mx);
@@ -1748,10 +1749,12 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
     }
   };
 
-  // ---- tile t from buffer BUF = t % 2
-  auto tile_body = [&](auto bufc, int t) __attribute__((always_inline)) {
+  // ---- tile t from buffer BUF = t % 2. FIRST (t = 0): the exponent reference is the maximum of both halves, so
+  // that the tile's largest probability is 1 without rounding, and the first half's softmax waits for it
+  auto tile_body = [&](auto bufc, auto firstc, int t) __attribute__((always_inline)) {
     constexpr int BUF = decltype(bufc)::value;
-    if (t == 0) wait_vmcnt<0>(); else wait_vmcnt<1>();   // this wave's gathers of tile t
+    constexpr bool FIRST = decltype(firstc)::value;
+    if constexpr (FIRST) wait_vmcnt<0>(); else wait_vmcnt<1>();   // this wave's gathers of tile t
     if (zero_rows) {   // rare: rows out of range read as zeros
       wait_vmcnt<0>();
 #pragma unroll 1
@@ -1764,8 +1767,9 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
     uint4 af[KPF];
 #pragma unroll
     for (int j = 0; j < KPF; ++j) af[j] = k_frag(0, j, BUF);
+    if constexpr (!FIRST)
 #pragma unroll
-    for (int m = NPV - NPRE; m < NPV; ++m) pv(m);   // of tile t-1
+      for (int m = NPV - NPRE; m < NPV; ++m) pv(m);   // of tile t-1
     __builtin_amdgcn_sched_barrier(0);
     static_for<0, 2 * KS>([&](auto jc) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value, half = j / KS, ks = j % KS;
@@ -1779,13 +1783,21 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
         if constexpr (g < GPW - 1) gather_part(g, ix, BUF ^ 1);
         else ids_dma(t + 4);   // slot t % 4 held the ids of tile t, read two iterations ago
       }
-      if constexpr (half == 1 && (ks & 1) && ks / 2 < NST) smx(ks / 2, 0, t, c[0][0], c[0][1]);
+      if constexpr (!FIRST && half == 1 && (ks & 1) && ks / 2 < NST) smx(ks / 2, 0, t, c[0][0], c[0][1]);
       __builtin_amdgcn_sched_barrier(0);
     });
+    if constexpr (FIRST) {
+      smx(0, 1, t, c[1][0], c[1][1]);
+      const float m1 = max8();
+      smx(0, 0, t, c[0][0], c[0][1]);
+      m_used = max_half_swap(fmaxf(m1, max8())) * cpos;
+#pragma unroll
+      for (int st = 1; st < NST; ++st) smx(st, 0, t, c[0][0], c[0][1]);
+    }
     zero_rows = ix.zero_rows;
 #pragma unroll
     for (int m = KPF; m < VR; ++m) vb[m] = v_frag(m, BUF);
-    rescale();
+    if constexpr (!FIRST) rescale();
     static_for<0, ON>([&](auto mc) __attribute__((always_inline)) {
       constexpr int m = decltype(mc)::value;
       pv(m);
@@ -1794,7 +1806,7 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
       __builtin_amdgcn_sched_barrier(0);
     });
     ix = tile_idx(t + 2);
-    rescale();
+    if constexpr (!FIRST) rescale();   // (no half of the first tile exceeds its maximum)
 #pragma unroll
     for (int m = ON; m < NPV - NPRE; ++m) {
       pv(m);
@@ -1802,9 +1814,10 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  for (int t = 0; t < ntiles; t += 2) {
-    tile_body(std::integral_constant<int, 0>{}, t);
-    if (t + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, t + 1);
+  tile_body(std::integral_constant<int, 0>{}, std::true_type{}, 0);
+  for (int t = 1; t < ntiles; t += 2) {
+    tile_body(std::integral_constant<int, 1>{}, std::false_type{}, t);
+    if (t + 1 < ntiles) tile_body(std::integral_constant<int, 0>{}, std::false_type{}, t + 1);
   }
 #pragma unroll
   for (int m = NPV - NPRE; m < NPV; ++m) pv(m);

@@ -537,6 +537,32 @@ def test_two_wave_form_climbing_scores(dev, dtype):
     compare(out[:, :4], smax[:, :, :4], ssum[:, :, :4], *o, what=f"two-wave climbing {dtype}")
 
 
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_two_wave_form_largest_probability_is_exact(dev, dtype):
+    """The first tile's exponent reference is the maximum over its 32 tokens, not its first half: 300
+    rows of 16 heads whose tokens 16 .. 31 score d above tokens 0 .. 15 (d different for every row
+    and head, below the lazy rescaling's threshold). Then the 16-bit P of the upper tokens is exactly
+    1 and, with values 0 and 1, the output 1 / (1 + exp(-d)) holds up to its own rounding: half a
+    spacing of the type in [0.5, 1), and 1e-5 for the 32-bit sums."""
+    R, N1, D = 300, 16, 512
+    x = (torch.arange(R * N1) % 190 + 10).reshape(1, R, N1).float() / 64   # exact in both types
+    qr = torch.zeros(1, R, N1, 64)
+    qr[..., 0] = x
+    k, kr = torch.zeros(1, 32, 1, D), torch.zeros(1, 32, 1, 64)
+    k[:, 16:], kr[:, 16:, :, 0] = 1.0, 1.0
+    si = torch.arange(32, dtype=torch.int32).repeat(1, R, 1, 1)
+    to = lambda t: t.to(DT[dtype]).to(dev)
+    out, smax, ssum = sparse_flash_attention(to(torch.zeros(1, R, N1, D)), to(k), to(k), si.to(dev), scale_value=0.5,
+                                             query_rope=to(qr), key_rope=to(kr), sparse_mode=0,
+                                             return_softmax_lse=True)
+    torch.cuda.synchronize()
+    want = torch.sigmoid(x.double() * 0.5)
+    assert torch.equal(smax[0, 0].cpu(), x[0] * 0.5)
+    half = 2.0 ** (-12 if dtype == "fp16" else -9)
+    err = (out.double().cpu() - want[..., None]).abs().max().item()
+    assert err <= half + 1e-5, (err, half)
+
+
 @pytest.mark.parametrize("B", [24, 100, 129, 255])
 def test_decode_batches_that_do_not_divide_the_cus(dev, B):
     """Decode batches whose splits are rounded down to one round of work-groups (24: 4 splits of 512
