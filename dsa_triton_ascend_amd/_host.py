@@ -76,14 +76,14 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
-UPLOAD_MAX = 8192   # dsa_upload_i32's limit
+UPLOAD_MAX = 8192   # values a dsa_upload_i32 call takes
 
 
 def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | None = None, wait: bool = True):
     """The int32 length and offset arrays of a call on the device, views of one tensor (each padded
-    to 16 bytes), written by one launch on the current stream (dsa_upload_i32); `zero` (a
-    byte tensor) is cleared by the same launch. More values than a launch takes, or a device
-    that is not the current one, go by a copy. With `wait` the host waits until the arrays and
+    to 16 bytes), written on the current stream by dsa_upload_i32 (one launch up to 56 values, then
+    one per 960); `zero` (a byte tensor) is cleared by the first. For a device that is not the
+    current one they go by a copy. With `wait` the host waits until the arrays and
     all that the caller put on this stream before are in place: a kept plan may run on any
     stream, and these arrays bound its addresses. A call that builds its plan and runs it at
     once, on one stream, needs no wait. Under stream capture there is none to wait for: the
@@ -99,14 +99,18 @@ def upload(lib, device: torch.device, *arrays: list[int], zero: torch.Tensor | N
     except OverflowError as e:   # torch's error for such a value
         raise RuntimeError("value cannot be converted to type int32 without overflow") from e
     n = len(flat)
-    if n <= UPLOAD_MAX and device.index in (None, torch.cuda.current_device()):
+    if device.index in (None, torch.cuda.current_device()):
         t = torch.empty(n, dtype=torch.int32, device=device)
-        _lib.check(lib.dsa_upload_i32(flat.buffer_info()[0], n, t.data_ptr(), ptr(zero),
-                                      0 if zero is None else zero.numel(), stream_ptr(device)), "dsa_upload_i32")
+        src, dst, stream = flat.buffer_info()[0], t.data_ptr(), stream_ptr(device)
+        zero_ptr, zero_bytes = ptr(zero), 0 if zero is None else zero.numel()
+        for i in range(0, max(n, 1), UPLOAD_MAX):
+            _lib.check(lib.dsa_upload_i32(src + 4 * i, min(n - i, UPLOAD_MAX), dst + 4 * i, zero_ptr, zero_bytes,
+                                          stream), "dsa_upload_i32")
+            zero_ptr, zero_bytes = None, 0
     else:
         if zero is not None:
             zero.zero_()
-        t = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=True)
+        t = torch.frombuffer(flat, dtype=torch.int32).to(device) if n else torch.empty(0, dtype=torch.int32, device=device)
     if wait and not torch.cuda.is_current_stream_capturing():
         torch.cuda.current_stream(device).synchronize()
     return t.split(sizes)

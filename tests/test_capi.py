@@ -330,18 +330,27 @@ def test_upload_i32_rejects_bad_arguments():
     assert lib.dsa_upload_i32(p, 0, None, None, 0, None) == _lib.DSA_OK   # nothing to do: no launch
 
 
-@pytest.mark.parametrize("n", [3, 9000])
+@pytest.mark.parametrize("n,device", [(3, "cpu"), (8192, "cpu"), (8196, "cpu"), (20000, "cpu"), (5, "cpu:1")])
 @pytest.mark.parametrize("wait", [True, False])
-def test_upload_wait_and_capture(monkeypatch, n, wait):
+def test_upload_wait_and_capture(monkeypatch, n, device, wait):
     """A kept plan's arrays are in place when its constructor returns (its run() may be on another
-    stream): the wait follows the launch, or the copy that large arrays take, and the clearing.
-    Under stream capture the launch is recorded and nothing waits."""
+    stream): the wait follows the calls of at most 8192 values each, of which the first clears
+    the prefix, or the copy for a device that is not the current one. Under stream capture the
+    calls are recorded and nothing waits."""
     from dsa_triton_ascend_amd import _host as H
-    done = []
+    done, out, base = [], [0] * (n + 3), [0]
+    empty = torch.empty
+
+    def first_tensor(*a, **k):
+        t = empty(*a, **k)
+        base[0] = t.data_ptr()
+        return t
 
     class Lib:
-        def dsa_upload_i32(self, *a):
-            done.append("launch")
+        def dsa_upload_i32(self, host, count, dst, zero, zero_bytes, stream):
+            done.append((count, zero_bytes))
+            at = (dst - base[0]) // 4
+            out[at:at + count] = ctypes.cast(host, ctypes.POINTER(ctypes.c_int32))[:count]
             return 0
 
     class Stream:
@@ -363,22 +372,26 @@ def test_upload_wait_and_capture(monkeypatch, n, wait):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(H, "stream_ptr", lambda device: 7)
-    values = list(range(n))
-    (got,) = H.upload(Lib(), torch.device("cpu"), values, zero=Zero(), wait=wait)
-    assert done == (["launch"] if n <= H.UPLOAD_MAX else ["zero"]) + ["wait"] * wait
-    if n > H.UPLOAD_MAX:
+    monkeypatch.setattr(torch, "empty", first_tensor)
+    values, padded = list(range(n)), (n + 3) // 4 * 4
+    got = H.upload(Lib(), torch.device(device), values, zero=Zero(), wait=wait)[0]
+    if device == "cpu":
+        calls = [(min(8192, padded - i), 16 if i == 0 else 0) for i in range(0, padded, 8192)]
+        assert out[:n] == values
+    else:
+        calls = ["zero"]
         assert got[:n].tolist() == values
-    if n <= H.UPLOAD_MAX:
-        capturing[0], done[:] = True, []
-        H.upload(Lib(), torch.device("cpu"), values, wait=wait)
-        assert done == ["launch"]
+    assert done == calls + ["wait"] * wait
+    capturing[0], done[:] = True, []
+    H.upload(Lib(), torch.device(device), values, zero=Zero(), wait=wait)
+    assert done == calls
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("counts", [(1, 0, 3, 1), (14, 14, 14, 14), (57,), (960,), (961, 2), (8192,), (8193, 5)])
+@pytest.mark.parametrize("counts", [(1, 0, 3, 1), (14, 14, 14, 14), (57,), (960,), (961, 2), (8192,), (8193, 5), (2500,) * 4, (17000, 3)])
 def test_upload_of_length_arrays(counts):
     """The call's length arrays at the edges of the launch's sizes (56 and 960 values a launch, 8192
-    a call, a copy above), padded to 16 bytes each, with the workspace prefix cleared beside them."""
+    a call), padded to 16 bytes each, with the workspace prefix cleared beside them."""
     from dsa_triton_ascend_amd import _host as H
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
