@@ -162,7 +162,8 @@ class AttentionPlan:
                 self.out.data_ptr(), H.ptr(self.sm_max), H.ptr(self.sm_sum), self.ws.data_ptr(),
                 self.ws_bytes, self.kv_splits, H.stream_ptr(self.dev)), "dsa_sfa_fwd")
         if not self.return_lse:
-            z = torch.zeros((2,) + self.sm_shape, dtype=torch.float32, device=self.dev)
+            z = [torch.empty(self.sm_shape, dtype=torch.float32, device=self.dev) for _ in range(2)]
+            torch._foreach_zero_(z)   # one launch for both
             return self.out, z[0], z[1]
         return self.out, self.sm_max, self.sm_sum
 

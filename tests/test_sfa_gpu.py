@@ -185,6 +185,18 @@ def test_lse_not_requested_gives_zeros(dev):
     assert not smax.any() and not ssum.any() and out.abs().sum() > 0
 
 
+def test_zero_statistics_share_no_storage(dev):
+    """Without return_softmax_lse the two zero tensors are the caller's own, each with its storage
+    (an odd element count: a second half would start unaligned)."""
+    q, k, v, qr, kr = _inputs(1, 3, 64, 1, 128, "bf16")
+    si = _ref_indices(1, 3, 64, 16, 1, 3)
+    _, smax, ssum = sparse_flash_attention(q.to(dev), k.to(dev), v.to(dev), torch.from_numpy(si).to(dev),
+                                           scale_value=0.1, query_rope=qr.to(dev), key_rope=kr.to(dev), sparse_mode=3)
+    for t in (smax, ssum):
+        assert t.shape == (1, 1, 3, 1) and t.data_ptr() % 16 == 0 and not t.any()
+        assert t.storage_offset() == 0 and t.untyped_storage().nbytes() == 4 * t.numel()
+
+
 def test_tnd(dev):
     lens_q, lens_k = [5, 1, 40, 17], [64, 9, 40, 100]
     N1, D, count = 16, 512, 32
