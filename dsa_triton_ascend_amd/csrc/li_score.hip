@@ -413,22 +413,22 @@ __global__ __launch_bounds__(NW * 64) void li_score_kernel(LiScoreArgs a) {
 }
 
 // ---------------------------------------------------------------- few query rows (decode)
-// Batches of at most ROWS_MAX query rows (a decode step, with speculative tokens a few): the
-// call reads every key once for one or a few rows, so it is bound by HBM (256 bytes a key against
-// 32 MFMA cycles), and the kernel above keeps one of its eight waves busy there. Here a
+// Batches of one or two query rows (a decode step, with or without a speculative token): the
+// call reads every key once for one or two rows, so it is bound by HBM (256 bytes a key against
+// 32 MFMA cycles), and the kernel above keeps one or two of its eight waves busy there. Here a
 // work-group (four waves) takes `chunk` keys of one row and its waves take the chunk's 32-key
 // subtiles in turn, each on its own: a wave copies a subtile (8 KB) into one of its two LDS
 // buffers while it computes the one before, so no barrier couples the waves and eight waves keep
 // 64 KB a CU in flight. The Q fragments (G <= 64) stay in VGPRs. Chunks are cut from the row's
-// own visible length, so sequences of uneven lengths leave no work-group with a long one; the
-// rows of one batch are dispatched 8 work-groups apart, on one XCD, whose L2 then serves the
-// second row's keys, and the chunk an XCD starts with turns with the batch (the last chunks of
-// short sequences are empty: without the turn the XCDs that take them idle, 48 -> 38 us for 200
-// sequences of 300 .. 6000 tokens). Same products, sums and rounding order as above.
-// 64 sequences of 4K .. 32K tokens (302 MB of keys), against the kernel above: 118 -> 60.5 us
-// (5.0 TB/s; a large copy moves 4.9). The rows of one batch share no registers, so their cost adds
-// up: 2 rows each 125 -> 96 us, 3 rows 134 -> 110, 4 rows 144 -> 130; from 5 on the kernel above.
-constexpr int ROWS_MAX = 4;
+// own visible length, so sequences of uneven lengths leave no work-group with a long one. The
+// (batch, chunk) pairs are dealt round the XCDs in groups of eight, a pair's two rows 8 work-groups
+// apart, on one XCD, whose L2 then serves the second row's keys; the chunk a batch starts with
+// turns with the batch (the last chunks of short sequences are empty: without the turn the XCDs
+// that take them idle, 64 sequences of 1K .. 8K tokens 18.9 -> 15.3 us).
+// Same products, sums and rounding order as above. Against that kernel, one row each: 64 sequences of
+// 4K .. 32K tokens (253 MB of keys, paged) 120 -> 48.8 us (5.2 TB/s; a large copy moves 4.9); 64 of 8192
+// 31.0 -> 23.9; 300 of 128 9.3 -> 7.2; 512 of 4096 118 -> 99. Two rows, the same 64 sequences: 126 -> 59.
+constexpr int ROWS_MAX = 2;
 constexpr int ROWS_NW = 4;            // waves per work-group
 constexpr int ROWS_CHUNK_MAX = 2048;  // keys per work-group
 
@@ -440,14 +440,18 @@ __global__ __launch_bounds__(ROWS_NW * 64, 2) void li_score_rows_kernel(LiScoreA
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = blockIdx.z, n2 = blockIdx.y;
-  // blockIdx.x = (group of 8 chunks, row, chunk of the group)
+  const int n2 = blockIdx.y;
+  // blockIdx.x = (group of 8 items, row, item of the group), item = (batch, chunk)
   const int R = a.max_rows_per_batch;
   const int x8 = (int)blockIdx.x >> 3;
-  const int ch = (x8 / R) * 8 + (((int)blockIdx.x + b) & 7), s1 = x8 % R;
+  const int g8 = x8 / R, s1 = x8 - g8 * R;
+  const int item = g8 * 8 + ((int)blockIdx.x & 7);
+  const int b = item / nchunk;
+  if (b >= a.batch) return;
+  const int ch = (item - b * nchunk + b) % nchunk;
   const int rows_b = a.row_start[b + 1] - a.row_start[b];
   const int aq = a.act_q[b], ak = a.act_k[b];
-  if (ch >= nchunk || s1 >= rows_b || s1 >= aq) return;
+  if (s1 >= rows_b || s1 >= aq) return;
   const int L = visible_len(s1, aq, ak, a.s2, a.sparse_mode);
   int c0 = ch * chunk;
   if (c0 >= L) return;
@@ -606,21 +610,44 @@ __global__ __launch_bounds__(ROWS_NW * 64, 2) void li_score_rows_kernel(LiScoreA
   }
 }
 
-template <int IO, bool PAGED>
-void launch_rows(const LiScoreArgs& a, hipStream_t s, int MT) {
-  // keys per work-group: the largest of 256 .. 2048 with at least 384 work-groups at the longest
-  // length (the others are shorter by an unknown share, and a CU holds two). Fewer, longer ones
-  // spare Q loads and prologues: 64 sequences of 4K .. 32K, 2048 keys 60.5 us, 1024 67, 512 72;
-  // 200 of 300 .. 6000, 2048 39, 512 49; 8 of 3K .. 60K, 1024 16.9, 512 19.7, 256 22; one of
-  // 100000, 256 9.0, 128 13.1.
+// Keys per work-group: the largest of 256 .. 2048 with at least 384 work-groups at the longest
+// length (the others are shorter by an unknown share, and a CU holds two). Fewer, longer ones
+// spare Q loads and prologues: 64 sequences of 8192, 2048 keys 22.9 us, 1024 23.6, 512 24.6; 64 of
+// 1K .. 8K, 2048 15.1, 512 16; 8 of 32768, 1024 14.2, 512 15; one of 100000, 512 7.8, 1024 9.4.
+struct RowsShape {
+  int chunk, nchunk;
+  int64_t blocks;   // gridDim.x
+};
+inline RowsShape rows_shape(const LiScoreArgs& a) {
   const int64_t rows = (int64_t)a.max_rows_per_batch * a.n2 * a.batch;
   const int kv = a.max_kv > 0 ? a.max_kv : 1;
   int chunk = ROWS_CHUNK_MAX;
   while (chunk > 256 && rows * ((kv + chunk - 1) / chunk) < 384) chunk >>= 1;
   const int nchunk = (kv + chunk - 1) / chunk;
-  const dim3 grid((unsigned)((nchunk + 7) / 8 * 8 * a.max_rows_per_batch), a.n2, a.batch), block(ROWS_NW * 64);
-  if (MT == 1) hipLaunchKernelGGL((li_score_rows_kernel<IO, 1, PAGED>), grid, block, 0, s, a, chunk, nchunk);
-  else hipLaunchKernelGGL((li_score_rows_kernel<IO, 2, PAGED>), grid, block, 0, s, a, chunk, nchunk);
+  return {chunk, nchunk, ((int64_t)nchunk * a.batch + 7) / 8 * 8 * a.max_rows_per_batch};
+}
+
+// Whether the few-row kernel takes the call. One row a batch: always (it was the faster one at each of
+// 1 .. 1000 sequences of 128 .. 100000 keys, by 5% to 9x). Two rows: where a sequence has more than a
+// few subtiles, else its second work-group costs more than the shared read saves (512 sequences of
+// 128 keys 11.6 us in the kernel above, 13.5 here; 256 of 500 12.0 against 11.3), and, on contiguous keys,
+// up to 400 MB of them (512 of 4096, 537 MB: 122.6 against 130.7; 256 of 6000, 393 MB: 96.7 against 94.2;
+// paged, whose page lookups cost the other more, 147 against 135). Three and more: the kernel above (64
+// sequences of 8192 keys, three rows 30.8 against 41, four 35.1 against 46.9).
+inline bool use_rows(const LiScoreArgs& a) {
+  if (a.max_rows_per_batch > ROWS_MAX) return false;
+  if (rows_shape(a).blocks >= (1 << 24)) return false;   // a launch's threads are counted in 32 bits
+  if (a.max_rows_per_batch == 1) return true;
+  const int64_t bytes = (int64_t)a.batch * a.n2 * a.max_kv * 256;
+  return a.max_kv > 384 && (a.block_table || bytes <= 400 * 1000 * 1000);
+}
+
+template <int IO, bool PAGED>
+void launch_rows(const LiScoreArgs& a, hipStream_t s, int MT) {
+  const RowsShape p = rows_shape(a);
+  const dim3 grid((unsigned)p.blocks, a.n2), block(ROWS_NW * 64);
+  if (MT == 1) hipLaunchKernelGGL((li_score_rows_kernel<IO, 1, PAGED>), grid, block, 0, s, a, p.chunk, p.nchunk);
+  else hipLaunchKernelGGL((li_score_rows_kernel<IO, 2, PAGED>), grid, block, 0, s, a, p.chunk, p.nchunk);
 }
 
 template <int IO, int D, bool PAGED>
@@ -635,7 +662,7 @@ void launch_mt(const LiScoreArgs& a, hipStream_t s, int MT, dim3 grid, dim3 bloc
 template <int IO, int D>
 hipError_t launch_d(const LiScoreArgs& a0, hipStream_t s, int MT) {
   LiScoreArgs a = a0;
-  if (D == 128 && MT <= 2 && a.max_rows_per_batch <= ROWS_MAX) {
+  if (D == 128 && MT <= 2 && use_rows(a)) {
     if (a.block_table) launch_rows<IO, true>(a, s, MT);
     else launch_rows<IO, false>(a, s, MT);
     return hipGetLastError();

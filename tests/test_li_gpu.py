@@ -450,10 +450,50 @@ def test_topk_instances_by_rows_and_length(dev, S1, S2, K, family):
     test_topk_crafted_score_rows(dev, S1, S2, K, family)
 
 
+@pytest.mark.parametrize("B,S1,lens,N2", [(300, 1, (1, 128), 1), (13, 1, (400, 2500), 2), (70, 2, (380, 520), 1),
+                                          (5, 2, (2000, 2300), 3), (33, 2, (384, 384), 1), (9, 2, (385, 385), 1),
+                                          (100, 1, (2100, 6000), 1)])
+@pytest.mark.parametrize("page", [None, 32])
+def test_few_query_rows_work_group_order(dev, B, S1, lens, N2, page):
+    """The few-row kernel's order of work-groups ((batch, chunk) pairs in groups of eight, a pair's rows
+    8 apart): one chunk a batch, chunk counts that 8 does not divide, pairs past the last
+    batch, and the line between the kernels (384 keys at two rows). Scores with G = 1 head of
+    weight 1 and small whole numbers are exact, so every score is compared with the CPU's."""
+    from dsa_triton_ascend_amd.lightning_indexer import IndexerPlan
+    rng = np.random.RandomState(7)
+    D, cap = 128, max(lens)
+    ak = rng.randint(lens[0], lens[1] + 1, B).tolist()
+    ak[0] = cap
+    q = torch.from_numpy(rng.randint(-2, 3, (B, S1, N2, D)).astype(np.float32))
+    k = torch.from_numpy(rng.randint(-1, 2, (B, cap, N2, D)).astype(np.float32))
+    w = torch.ones(B, S1, N2)
+    if page is None:
+        plan = IndexerPlan(q.half().to(dev), k.half().to(dev), w.to(dev), None, ak, sparse_count=64)
+    else:
+        mb = (cap + page - 1) // page
+        pad = torch.zeros(B, mb * page, N2, D)
+        pad[:, :cap] = k
+        perm = torch.from_numpy(rng.permutation(B * mb).astype(np.int32))
+        cache = torch.empty(B * mb, page, N2, D, dtype=torch.float16)
+        cache[perm.long()] = pad.reshape(B * mb, page, N2, D).half()
+        plan = IndexerPlan(q.half().to(dev), cache.to(dev), w.to(dev), None, ak, perm.reshape(B, mb).to(dev),
+                           layout_key="PA_BSND", sparse_count=64)
+    plan.scores.fill_(0x7E00)   # NaN pattern
+    plan.score()
+    torch.cuda.synchronize()
+    got = plan.scores.view(torch.float16).cpu().reshape(B, S1, N2, -1)
+    for b in range(B):
+        want = torch.relu(torch.einsum("snd,knd->snk", q[b], k[b, :ak[b]]))
+        for s in range(S1):
+            L = max(ak[b] - S1 + s + 1, 0)
+            assert torch.equal(got[b, s, :, :L].float(), want[s, :, :L]), (b, s)
+            assert torch.isnan(got[b, s, :, L:]).all(), (b, s)
+
+
 @pytest.mark.parametrize("S1,N1,N2", [(1, 64, 1), (2, 8, 1), (3, 80, 2), (4, 33, 1), (5, 64, 1)])
 @pytest.mark.parametrize("page", [None, 16, 48, 64])
 def test_few_query_rows(dev, S1, N1, N2, page):
-    """One to four query rows a batch (decode; five take the general kernel): key counts at the
+    """One and two query rows a batch (decode) and a few more (the general kernel): key counts at the
     edges of the 32-key subtile and of the work-group's chunk, several key heads, partial head
     tiles, pages smaller and larger than a subtile with a missing one, each score against the
     oracle."""
