@@ -31,6 +31,7 @@
 //    next tile; fully causal-masked tiles are never loaded or computed;
 //  * row blocks are issued heaviest-first (largest s1 first) to flatten the
 //    causal triangle's tail.
+#include <cmath>
 #include <type_traits>
 
 #include "dsa_common.hpp"
@@ -659,6 +660,45 @@ void launch_mt(const LiScoreArgs& a, hipStream_t s, int MT, dim3 grid, dim3 bloc
   }
 }
 
+// Number of work-groups over which a row block's keys are split (tiles of bn keys), so that few row
+// blocks fill the chip: the split with the shortest modelled time. Only max_kv is known here.
+//  * Q in registers (qreg): one work-group a CU; each costs about 10 tiles of 64 keys besides its own (Q,
+//    the first tiles' latency). The time is at least the longest work-group's, the mean work's over 256
+//    CUs, and that of whole rounds of the shortest ones (under a causal mask the row blocks see between
+//    max_kv - rows and max_kv keys). With several sequences 3 parts of 10 go to the case that they hold
+//    half of max_kv on average and later work-groups fill the gaps.
+//  * Q read from L2 again for every tile (more than 64 heads a key head): a split costs half a tile, and ten
+//    or more keep a work-group's keys small enough for its XCD's L2.
+// Against at most 16 splits towards 512 work-groups: 512 rows of 4096 keys 37.7 -> 31.0 us (4 splits), 64 of
+// 16000 26.1 -> 18.4 (32), 8 of 100000, one sequence, 75 -> 11.2 (256); paged, 64 sequences of 4096, 5 rows,
+// 38.8 -> 32.7 (4), 100 of 3000, 8 rows, 61.1 -> 47.5 (2); 128 heads, 512 rows of 4096 798 -> 279 (16).
+inline int key_split(const LiScoreArgs& a, int bn, bool qreg) {
+  const int64_t blocks = (int64_t)((a.max_rows_per_batch + NW - 1) / NW) * a.n2 * a.batch;
+  const int tiles = a.max_kv > 0 ? (a.max_kv - 1) / bn + 1 : 0;
+  const int cap = qreg || blocks == 0 ? 256 : (int)(blocks < 8 ? 256 / blocks : 32);
+  const int most = tiles < cap ? tiles : cap;
+  const int least = qreg ? 1 : (tiles < 10 ? tiles : 10);
+  const float over = qreg ? (bn > 64 ? 5.f : 10.f) : 0.5f;
+  const int hidden = a.sparse_mode == 3 ? (a.max_rows_per_batch < a.max_kv ? a.max_rows_per_batch : a.max_kv) : 0;
+  const float shortest = qreg ? (float)(a.max_kv - hidden) / bn : (float)tiles, mean = (tiles + shortest) / 2;
+  float best = INFINITY;
+  int pick = 1, last = 0;
+  for (int ks = least > 0 ? least : 1; ks <= most; ++ks) {
+    const int piece = (tiles + ks - 1) / ks;
+    if (piece == last) continue;   // more work-groups, none shorter
+    last = piece;
+    const float longest = piece + over, rounds = (float)((blocks * ks + 255) / 256);
+    const float even = fmaxf(fmaxf(longest, blocks * (mean + over * ks) / 256), rounds * ((qreg ? shortest / ks : piece) + over));
+    const float uneven = fmaxf(longest, blocks * (mean / 2 + over * ks) / 256);
+    const float t = qreg && a.batch > 1 ? 0.7f * even + 0.3f * uneven : even;
+    if (t < best) {
+      best = t;
+      pick = ks;
+    }
+  }
+  return pick;
+}
+
 template <int IO, int D>
 hipError_t launch_d(const LiScoreArgs& a0, hipStream_t s, int MT) {
   LiScoreArgs a = a0;
@@ -667,31 +707,7 @@ hipError_t launch_d(const LiScoreArgs& a0, hipStream_t s, int MT) {
     else launch_rows<IO, false>(a, s, MT);
     return hipGetLastError();
   }
-  // Short query batches leave CUs idle: split each row block's keys over ks work-groups. The
-  // registers hold one work-group a CU, and each costs about OVER tiles besides its own (Q, the
-  // first tiles' latency), so ks is the one with the shortest makespan: rounds of 256 equal
-  // work-groups where all rows see about the same keys, and under a causal triangle (rows up to
-  // half as many as keys and more) or over paged sequences of uneven lengths the mean work or the
-  // longest block, whichever is larger.
-  // B=1, 512 rows of 4096 keys: ks = 8 (two rounds) 41.5 us, 4 (one) 33.0; 64 rows of 16000: 16
-  // 27.3, 32 19.8; 4 x 300 rows of 5000: 4 105, 3 92; 2048 rows of 2048: 1 50, 2 40, 3 48.
-  constexpr int64_t OVER = 10;
-  const int64_t blocks = (int64_t)((a.max_rows_per_batch + NW - 1) / NW) * a.n2 * a.batch;
-  const int64_t tiles = (a.max_kv + LiTile<D>::BN - 1) / LiTile<D>::BN;
-  const bool causal = a.sparse_mode == 3 && 2 * (int64_t)a.max_rows_per_batch > a.max_kv;
-  const int64_t mean = causal ? tiles - (a.max_rows_per_batch / 2) / LiTile<D>::BN
-                      : a.block_table ? (tiles * 5 + 7) / 8 : tiles;
-  int64_t best = INT64_MAX;
-  a.key_split = 1;
-  for (int ks = 1; ks <= 64 && ks <= tiles; ++ks) {
-    const int64_t longest = (tiles + ks - 1) / ks + OVER;
-    const int64_t sum = blocks * (mean + OVER * ks) / 256;
-    const int64_t t = causal || a.block_table ? (sum > longest ? sum : longest) : (blocks * ks + 255) / 256 * longest;
-    if (t < best) {
-      best = t;
-      a.key_split = ks;
-    }
-  }
+  a.key_split = key_split(a, LiTile<D>::BN, MT <= 2 && MT * D <= 512);
   dim3 grid((unsigned)(((a.max_rows_per_batch + NW - 1) / NW) * a.key_split), a.n2, a.batch), block(NW * 64);
   if (a.block_table)
     launch_mt<IO, D, true>(a, s, MT, grid, block);

@@ -7,6 +7,8 @@ size-independent invariants are checked on every row. Parity rule: see
 tests/parity.py (bit-exact ordered indices and values, except bf16/fp16
 rounding flips of scores within accumulation noise of a rounding midpoint).
 """
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -488,6 +490,48 @@ def test_few_query_rows_work_group_order(dev, B, S1, lens, N2, page):
             L = max(ak[b] - S1 + s + 1, 0)
             assert torch.equal(got[b, s, :, :L].float(), want[s, :, :L]), (b, s)
             assert torch.isnan(got[b, s, :, L:]).all(), (b, s)
+
+
+@pytest.mark.parametrize("B,S1,S2,N1,D", [(1, 9, 20000, 4, 128),      # 2 row blocks, 128 splits of a few tiles
+                                          (1, 300, 300, 4, 128),      # triangle: row blocks with fewer tiles than splits
+                                          (3, 5, 70, 4, 64), (2, 40, 3000, 4, 96), (2, 24, 1500, 4, 256),
+                                          (1, 64, 1300, 128, 128), (2, 17, 330, 72, 128),   # Q not in registers
+                                          (1, 40, 900, 16, 512)])
+@pytest.mark.parametrize("page", [None, 64])
+def test_key_splits(dev, B, S1, S2, N1, D, page):
+    """The general kernel's keys over many work-groups: every visible key is scored once whatever the
+    split (more splits than a row block has tiles among them), nothing past it is written. Three heads
+    of weight 1 and small whole numbers make the scores exact."""
+    from dsa_triton_ascend_amd.lightning_indexer import IndexerPlan
+    rng = np.random.RandomState(8)
+    ak = [S2] + rng.randint(S1, S2 + 1, B - 1).tolist()
+    q = torch.from_numpy(rng.randint(-1, 2, (B, S1, N1, D)).astype(np.float32))
+    k = torch.from_numpy(rng.randint(-1, 2, (B, S2, 1, D)).astype(np.float32))
+    w = torch.zeros(B, S1, N1)
+    heads = [0, N1 // 2, N1 - 1]
+    w[:, :, heads] = 1.0
+    if page is None:
+        plan = IndexerPlan(q.half().to(dev), k.half().to(dev), w.to(dev), None, ak, sparse_count=64)
+    else:
+        mb = (S2 + page - 1) // page
+        pad = torch.zeros(B, mb * page, 1, D)
+        pad[:, :S2] = k
+        perm = torch.from_numpy(rng.permutation(B * mb).astype(np.int32))
+        cache = torch.empty(B * mb, page, 1, D, dtype=torch.float16)
+        cache[perm.long()] = pad.reshape(B * mb, page, 1, D).half()
+        plan = IndexerPlan(q.half().to(dev), cache.to(dev), w.to(dev), None, ak, perm.reshape(B, mb).to(dev),
+                           layout_key="PA_BSND", sparse_count=64)
+    plan.scores.fill_(0x7E00)   # NaN pattern
+    plan.score()
+    torch.cuda.synchronize()
+    got = plan.scores.view(torch.float16).cpu().reshape(B, S1, -1).float()
+    for b in range(B):
+        dots = torch.relu(q[b][:, heads].reshape(-1, D) @ k[b, :ak[b], 0].t()).reshape(S1, 3, -1).sum(1)
+        seen = torch.arange(got.shape[2])[None] < (ak[b] - S1 + torch.arange(S1)[:, None] + 1)
+        want = torch.full_like(got[b], math.nan)
+        want[:, :ak[b]] = dots
+        want[~seen] = math.nan
+        assert torch.equal(got[b].nan_to_num(-1), want.nan_to_num(-1)), b
 
 
 @pytest.mark.parametrize("S1,N1,N2", [(1, 64, 1), (2, 8, 1), (3, 80, 2), (4, 33, 1), (5, 64, 1)])
