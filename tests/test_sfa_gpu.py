@@ -419,8 +419,8 @@ def test_forced_kv_splits_with_empty_splits(dev, kv_splits):
 @pytest.mark.parametrize("kv_splits", [2, 5])
 def test_forced_kv_splits_block_size_2(dev, N1, kv_splits):
     """KV splits over token lists built by the token-list launch (sparse_block_size 2): at
-    D = 512 the 8-wave attention forms (N1 <= 64, and N1 = 128) write the split
-    partials and the merge combines them, including splits past a short row's tokens."""
+    D = 512 and few work-groups the eight-wave form (N1 <= 64) or the four-wave one (N1 = 128) writes the
+    split partials and the merge combines them, including splits past a short row's tokens."""
     B, S1, S2, D, count, bs = 1, 8, 160, 512, 48, 2
     q, k, v, qr, kr = _inputs(B, S1, S2, N1, D, "bf16", seed=23)
     si = _ref_indices(B, S1, S2, count, bs, 3, seed=6)
@@ -530,6 +530,31 @@ def test_two_wave_form_rows_of_every_length(dev, N1, dtype, scale):
     o = SFA.sparse_flash_attention(_np(q), _np(cache), None, si, block_table=bt, query_rope=_np(qr),
                                    key_rope=_np(rcache), io_dtype=dtype, **kw)
     compare(out, smax, ssum, *o, what=f"two-wave N1={N1} {dtype} scale={scale}")
+
+
+@pytest.mark.parametrize("N1,dtype", [(16, "bf16"), (64, "fp16")])
+@pytest.mark.parametrize("S1,S2,kv_splits", [(140, 140, 2), (60, 200, 5)])
+def test_two_wave_form_split_partials(dev, N1, dtype, S1, S2, kv_splits):
+    """The two-wave form on KV splits (forced; sparse_block_size 2, so the token lists come from their
+    launch; more than 256 work-groups): partials and statistics of the splits that hold tokens, rows so
+    short that one split holds all (it writes the output itself) or the later ones are empty, and a
+    row without tokens."""
+    B, D, count, bs = 1, 512, S2 // 2, 2
+    assert S1 * kv_splits > 256
+    q, k, _, qr, kr = _inputs(B, S1, S2, N1, D, dtype, seed=24)
+    si = _ref_indices(B, S1, S2, count, bs, 3, seed=25)
+    si[0, 30, 0, :] = -1
+    for s1, n in ((20, 1), (40, 16), (50, 17), (55, 33)):   # 2, 32, 34 and 66 tokens where visible
+        si[0, s1, 0, n:] = -1
+    out, smax, ssum = sparse_flash_attention(q.to(dev), k.to(dev), k.to(dev), torch.from_numpy(si).to(dev),
+                                             scale_value=0.05, query_rope=qr.to(dev), key_rope=kr.to(dev),
+                                             sparse_block_size=bs, sparse_mode=3, return_softmax_lse=True,
+                                             kv_splits=kv_splits)
+    torch.cuda.synchronize()
+    o = SFA.sparse_flash_attention(_np(q), _np(k), None, si, 0.05, None, None, None, _np(qr), _np(kr), bs,
+                                   "BSND", "BSND", 3, True, io_dtype=dtype)
+    assert not out[0, 30].any()
+    compare(out, smax, ssum, *o, what=f"two-wave N1={N1} {dtype} S1={S1} kv_splits={kv_splits}")
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
