@@ -60,8 +60,8 @@ const char* dsa_last_error(void);
  * arguments: the host neither waits for the stream nor needs `host` to outlive the call,
  * and the call may be captured (the values are then part of the graph). Also clears
  * zero_bytes (a multiple of 16) at zero_dst, 16-byte aligned, if zero_dst is not NULL. For
- * the small length and offset arrays the entry points below take; n <= 8192
- * (DSA_ERR_UNSUPPORTED above: use a copy). No counterpart in the reference.
+ * the small length and offset arrays the entry points below take: one launch up to 56
+ * values, then one per 960; n <= 8192 (DSA_ERR_UNSUPPORTED above: several calls, or a copy). No counterpart in the reference.
  */
 int dsa_upload_i32(const int32_t* host, int n, int32_t* dst, void* zero_dst, size_t zero_bytes, void* stream);
 
