@@ -6,11 +6,11 @@
 // and quantised score), the other slots get -1 / 0. The reference's device
 // path calls mint.topk / mint.sort here (lightning_indexer_triton.py:343-361).
 //
-// One 256-thread work-group per score row (any length: indices are 32-bit):
-//   1. Thread t owns the contiguous index range [32t, 32t+32) of the row; the
-//      16-bit scores are mapped to order-preserving keys u (ord16) and kept in
-//      VGPRs as packed pairs (rows longer than 8192 entries are streamed from
-//      memory instead, in chunks of 8192). Waves holding no entry of the row skip
+// One work-group of TPB threads (256 or 1024) per score row (any length: indices are 32-bit):
+//   1. Thread t owns the contiguous index range [RPT t, RPT t + RPT) of the row (RPT 8 or
+//      32); the 16-bit scores are mapped to order-preserving keys u (ord16) and kept in
+//      VGPRs as packed pairs (rows longer than TPB * RPT entries are streamed from
+//      memory instead, in chunks of that many). Waves holding no entry of the row skip
 //      the per-entry loops below.
 //   2. L > k: a 2048-bin LDS histogram of u >> 5, scanned from the top bin, gives
 //      the bin holding the k-th largest key and the number of keys above that bin.
@@ -32,7 +32,9 @@
 //      scores, which is exactly the golden's tie rule.
 //   5. One pass writes the indices and 16-bit values in rank order.
 // The selection histogram and the sort's counters share one LDS array (they are
-// never live together), so a work-group needs ~16 KB and more of them fit a CU.
+// never live together): with 256 threads 8 KB of it and 1 KB of sort buffer per E (k = 2048:
+// 16 KB a work-group, eight of them fit a CU), with 1024 threads 32 KB and 4 KB per E (k = 4096:
+// 48 KB); WIDE adds another sort buffer's size.
 #include <type_traits>
 
 #include "dsa_common.hpp"
@@ -40,7 +42,7 @@
 namespace dsa {
 namespace {
 
-constexpr int ROW_CACHED = 8192;   // row entries that 256 threads hold in VGPRs, 32 each
+constexpr int ROW_CACHED_256 = 8192;   // row entries that 256 threads hold in VGPRs, 32 each
 
 __device__ __forceinline__ int visible_len(int s1, int aq, int ak, int S2, int mode) {
   int L;
@@ -255,9 +257,9 @@ __device__ __forceinline__ uint32_t block_scan_max2(uint32_t v, uint32_t m1, uin
   return off + x - v;
 }
 
-// SHORT: rows of at most ROW_CACHED entries (s2 <= 8192), held in registers in one chunk;
-// the chunked paths for longer rows are compiled out. Short rows with k <= 2048 are
-// compiled for eight waves per SIMD (64 VGPRs, 96 SGPRs: more SGPR spills to VGPR lanes,
+// SHORT: rows of at most TPB * RPT entries (2048, 8192 or 32768 in the instances below), held in
+// registers in one chunk; the chunked paths for longer rows are compiled out. With 256 threads,
+// short rows with k <= 2048 are compiled for eight waves per SIMD (64 VGPRs, 96 SGPRs: more SGPR spills to VGPR lanes,
 // which cost less than the latency an eighth work-group per CU hides). At eight waves per
 // SIMD the VALU issues for about two thirds of the kernel's time; LDS bank conflicts and
 // the chain of block barriers take most of the rest.
@@ -459,7 +461,7 @@ void li_topk_kernel(LiTopkArgs a) {
         }
       }
       compacted = true;
-    } else {   // rows longer than 8192 or a crowded bin: one more pass over the row
+    } else {   // rows of several chunks or a crowded bin: one more pass over the row
       resolve([&] {
 #pragma unroll 1
         for (int ch = 0; ch < nchunks; ++ch) {
@@ -509,7 +511,7 @@ void li_topk_kernel(LiTopkArgs a) {
   }
   if (!compacted) {
     // positions: selected-before = greater-before + min(ties-before, need); one scan of
-    // (greater << 16 | ties) per chunk (a chunk holds at most 8192 of each), which also
+    // (greater << 16 | ties) per chunk (a chunk holds at most TPB * RPT <= 32768 of each), which also
     // gives the largest and smallest key (the sort's pass range when every key is taken)
     uint32_t run_g = 0, run_e = 0;  // totals of previous chunks
     uint32_t kmax = 0, kmin_inv = 0;   // max of u, max of 0xFFFF - u over nonzero keys
@@ -817,7 +819,7 @@ hipError_t launch_li_topk(const LiTopkArgs& a, hipStream_t s) {
   // against 16.7) and for rows of several chunks (40000: 55 against 60), not between (512 rows of
   // 20000: 41.5 against 31.1).
   if (rows <= 512 && a.k <= 4096) {
-    if (a.s2 > dsa::ROW_CACHED && a.s2 <= 32768) return launch_topk_e<1024, 32, false, true, 4>(a, n, s);
+    if (a.s2 > dsa::ROW_CACHED_256 && a.s2 <= 32768) return launch_topk_e<1024, 32, false, true, 4>(a, n, s);
     if (rows <= 256) {
       if (a.s2 > 65536) return launch_topk_e<1024, 32, true, false, 4>(a, n, s);
       if (a.s2 > 32768) return launch_topk_e<1024, 32, false, false, 4>(a, n, s);
