@@ -830,6 +830,6 @@ hipError_t launch_li_topk(const LiTopkArgs& a, hipStream_t s) {
   // (256 rows of 256 entries: 10.7 -> 7.4 us; 1024 rows of 1500: 15.4 -> 12.2)
   if (a.s2 <= 2048 && a.k <= 2048) return launch_topk_e<256, 8, false, true, 8>(a, n, s);
   if (a.s2 > 65536) return launch_topk_e<256, 32, true, false, 64>(a, n, s);
-  if (a.s2 > dsa::ROW_CACHED) return launch_topk_e<256, 32, false, false, 64>(a, n, s);
+  if (a.s2 > dsa::ROW_CACHED_256) return launch_topk_e<256, 32, false, false, 64>(a, n, s);
   return launch_topk_e<256, 32, false, true, 64>(a, n, s);   // every visible row fits the registers
 }
