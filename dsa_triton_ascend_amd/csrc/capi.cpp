@@ -183,6 +183,22 @@ int dsa_li_topk(const uint16_t* scores, int64_t score_ld, int io_dtype, const in
   return hip_status(launch_li_topk(a, (hipStream_t)stream), "dsa_li_topk launch");
 }
 
+int dsa_li_topk_kv(const uint16_t* scores, int64_t score_ld, int io_dtype, const int32_t* row_start,
+                   const int32_t* act_q, const int32_t* act_k, int batch, int total_rows, int n2,
+                   int s2, int max_kv, int sparse_mode, int sparse_count, int32_t* indices,
+                   uint16_t* values, void* stream) {
+  const int st = check_li_topk("dsa_li_topk_kv", scores, score_ld, io_dtype, row_start, act_q, act_k, batch,
+                               total_rows, n2, s2, sparse_mode, sparse_count, indices);
+  if (st != DSA_OK) return st;
+  if (max_kv < 0) return fail(DSA_ERR_INVALID, "dsa_li_topk_kv: negative max_kv");
+  if (sparse_count > LI_TOPK_MAX_K)
+    return fail(DSA_ERR_UNSUPPORTED, "dsa_li_topk_kv: sparse_count=%d > %d (use dsa_li_topk_ws)", sparse_count,
+                LI_TOPK_MAX_K);
+  LiTopkArgs a{scores, score_ld, io_dtype, row_start, act_q, act_k, batch, total_rows, n2, s2,
+               sparse_mode, sparse_count, indices, values, max_kv};
+  return hip_status(launch_li_topk(a, (hipStream_t)stream), "dsa_li_topk_kv launch");
+}
+
 size_t dsa_li_topk_workspace_bytes(int total_rows, int n2, int s2, int sparse_count) {
   return li_topk_workspace_bytes(total_rows, n2, s2, sparse_count);
 }

@@ -408,6 +408,7 @@ struct LiTopkArgs {
   const int32_t* row_start; const int32_t* act_q; const int32_t* act_k;
   int batch, total_rows, n2, s2, sparse_mode, k;
   int32_t* idx; uint16_t* val;
+  int max_kv = 0;   // longest act_k the caller expects, 0: unknown (chooses the kernel, bounds nothing)
 };
 struct SfaArgs {
   const void* q; const void* qr; const void* k; const void* kr; int io;

@@ -818,12 +818,20 @@ hipError_t launch_li_topk(const LiTopkArgs& a, hipStream_t s) {
   // shorter throughput of 256 threads wins for rows that fit its registers (400 rows of 5000: 15.1
   // against 16.7) and for rows of several chunks (40000: 55 against 60), not between (512 rows of
   // 20000: 41.5 against 31.1).
-  if (rows <= 512 && a.k <= 4096) {
-    if (a.s2 > dsa::ROW_CACHED_256 && a.s2 <= 32768) return launch_topk_e<1024, 32, false, true, 4>(a, n, s);
-    if (rows <= 256) {
+  // S2 alone does not say how long the rows are: a paged cache's is the capacity of its block table.
+  // Rows that 256 threads hold in one chunk run faster there whatever S2 (S2 131072, 64 rows of 4096:
+  // 12.3 against 16.8 us; 32768, 500 rows of 1024: 11.3 against 21.7), longer ones from the first
+  // entry past it on the other side (16 rows of 8300: 23.0 against 12.4; 300: 26.1 against 23.3). A
+  // caller that does not say (max_kv 0) gets the long rows' form only up to 256 rows, where it
+  // loses least. Each instance is right for rows up to S2.
+  const int longest = a.max_kv > 0 && a.max_kv < a.s2 ? a.max_kv : a.s2;
+  if (a.k <= 4096) {
+    if (a.s2 <= dsa::ROW_CACHED_256) {
+      if (a.s2 > 2048 && rows <= 256) return launch_topk_e<1024, 8, false, true, 4>(a, n, s);
+    } else if (longest > dsa::ROW_CACHED_256 && rows <= (a.s2 <= 32768 && a.max_kv > 0 ? 512 : 256)) {
       if (a.s2 > 65536) return launch_topk_e<1024, 32, true, false, 4>(a, n, s);
       if (a.s2 > 32768) return launch_topk_e<1024, 32, false, false, 4>(a, n, s);
-      if (a.s2 > 2048) return launch_topk_e<1024, 8, false, true, 4>(a, n, s);
+      return launch_topk_e<1024, 32, false, true, 4>(a, n, s);
     }
   }
   // Short rows: eight entries a thread spread the per-entry loops over four times the threads

@@ -144,11 +144,11 @@ class IndexerPlan:
                 self.vals.data_ptr() if self.return_value else None, self.topk_ws.data_ptr(),
                 self.topk_ws.numel(), H.stream_ptr(self.dev)), "dsa_li_topk_ws")
             return
-        _lib.check(self.lib.dsa_li_topk(
+        _lib.check(self.lib.dsa_li_topk_kv(
             self.scores.data_ptr(), self.ld, self.io, self.d_row_start.data_ptr(),
             self.d_aq.data_ptr(), self.d_ak.data_ptr(), self.B, self.total_rows, self.N2, self.S2,
-            self.sparse_mode, self.k, self.idx.data_ptr(),
-            self.vals.data_ptr() if self.return_value else None, H.stream_ptr(self.dev)), "dsa_li_topk")
+            max(self.max_kv, 1), self.sparse_mode, self.k, self.idx.data_ptr(),
+            self.vals.data_ptr() if self.return_value else None, H.stream_ptr(self.dev)), "dsa_li_topk_kv")
 
     def run(self):
         self.score()

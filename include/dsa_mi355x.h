@@ -128,6 +128,16 @@ int dsa_li_topk(const uint16_t* scores, int64_t score_ld, int io_dtype,
                 int32_t* indices, uint16_t* values, void* stream);
 
 /*
+ * dsa_li_topk with the longest act_k that the caller expects (max_kv; 0: unknown). It only chooses the
+ * kernel: where S2 is a block table's capacity, sequences much shorter than it take another one. Same
+ * outputs, also for rows longer than max_kv (act_k written anew before a captured call runs again).
+ */
+int dsa_li_topk_kv(const uint16_t* scores, int64_t score_ld, int io_dtype,
+                   const int32_t* row_start, const int32_t* act_q, const int32_t* act_k,
+                   int batch, int total_rows, int n2, int s2, int max_kv, int sparse_mode,
+                   int sparse_count, int32_t* indices, uint16_t* values, void* stream);
+
+/*
  * Bytes of device workspace dsa_li_topk_ws needs: 0 for sparse_count <= 16384, else two
  * buffers of S2 8-byte entries per score row (total_rows * N2 * 16 * S2).
  */

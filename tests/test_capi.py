@@ -45,6 +45,10 @@ def test_invalid_arguments_return_status_without_gpu():
     assert st == _lib.DSA_ERR_UNSUPPORTED
     st = lib.dsa_li_topk(p, 70000, 1, p, p, p, 1, 1, 1, 70000, 3, 16385, p, None, None)
     assert st == _lib.DSA_ERR_UNSUPPORTED and b"16384" in lib.dsa_last_error()
+    st = lib.dsa_li_topk_kv(p, 70000, 1, p, p, p, 1, 1, 1, 70000, 512, 3, 16385, p, None, None)
+    assert st == _lib.DSA_ERR_UNSUPPORTED and b"16384" in lib.dsa_last_error()
+    st = lib.dsa_li_topk_kv(p, 70000, 1, p, p, p, 1, 1, 1, 70000, -1, 3, 64, p, None, None)
+    assert st == _lib.DSA_ERR_INVALID and b"max_kv" in lib.dsa_last_error()
     # above the LDS sort's cap: the workspace entry point sizes and checks its scratch
     assert lib.dsa_li_topk_workspace_bytes(4, 2, 70000, 16384) == 0
     assert lib.dsa_li_topk_workspace_bytes(4, 2, 70000, 16385) == 4 * 2 * 2 * 70000 * 8

@@ -564,3 +564,34 @@ def test_few_query_rows(dev, S1, N1, N2, page):
     check_topk_properties(gi.reshape(-1, K), gv.reshape(-1, K), Ls, K)
     stats = check_li(gi, gv, _np(q), dense, _np(w), np.full(B, S1), ak, K, 3, dtype)
     assert stats.flips <= max(4, 0.02 * stats.elements), stats
+
+
+@pytest.mark.parametrize("rows,pages,lens", [
+    (20, 600, (1, 9600, 513)), (20, 600, (1, 40, 8192)), (300, 600, (5, 8191, 4000)), (300, 600, (1, 8193, 300)),
+    (5, 2100, (7, 3000)), (5, 2100, (8193, 40)), (3, 4200, (1, 8192)), (3, 4200, (66000, 8200)), (520, 150, (9, 2400))])
+def test_topk_of_rows_shorter_than_the_capacity(dev, rows, pages, lens):
+    """Lengths far below the block table's capacity S2 (16 tokens a page) and on both sides of the 8192
+    entries at which the top-k changes its instance, bit for bit against the golden's stable sort; then
+    the lengths rewritten in place, beyond the longest that the plan was built with."""
+    from dsa_triton_ascend_amd.lightning_indexer import IndexerPlan
+    S2, K = 16 * pages, 512
+    kv = [lens[r % len(lens)] for r in range(rows)]
+    q = torch.zeros(rows, 1, 8, 128, dtype=torch.bfloat16, device=dev)
+    w = torch.zeros(rows, 1, 8, dtype=torch.float32, device=dev)
+    plan = IndexerPlan(q, torch.zeros(1, 16, 1, 128, dtype=torch.bfloat16, device=dev), w, actual_seq_lengths_key=kv,
+                       block_table=torch.zeros(rows, pages, dtype=torch.int32, device=dev), layout_key="PA_BSND",
+                       sparse_count=K, sparse_mode=3, return_value=True)
+    bits = _crafted_bits("wide", rows, S2, np.random.default_rng(12))
+    plan.scores[:rows, :S2] = torch.from_numpy(bits.view(np.int16)).to(dev)
+    vals = (bits.astype(np.uint32) << 16).view(np.float32)
+    for grown in (0, S2 - max(kv)):
+        plan.d_ak[:rows] += grown
+        plan.topk()
+        torch.cuda.synchronize()
+        gi, gv = plan.idx.reshape(rows, K).cpu().numpy(), plan.vals.reshape(rows, K).float().cpu().numpy()
+        for r in sorted({0, 1, 2, rows - 1} | set(range(0, rows, 97))):
+            L = min(kv[r] + grown, S2)
+            s = np.full(S2, -np.inf, np.float32)
+            s[:L] = vals[r, :L]
+            ei, ev = LI.select_topk(s, S2, K)
+            assert np.array_equal(gi[r], ei) and np.array_equal(gv[r], ev), (rows, S2, r, L, grown)
