@@ -1915,14 +1915,12 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hb = wave_u & 1, kq = wave_u >> 1;
   const int n1 = a.n1;
-  constexpr int h0 = 0;
-  const int hl = hb * 32 + (lane & 31);   // local head of this lane's S^T column
-  const int hs = h0 + hl;
+  const int hl = hb * 32 + (lane & 31);   // head of this lane's S^T column
   const int ntok_all = ws.counts[r];
   // Q^T fragments of k-steps 9 kq + j (nope, then rope), clamped heads zeroed below
   uint4 qf[w8::KQ];
   {
-    const int hc = hs < n1 ? hs : n1 - 1;
+    const int hc = hl < n1 ? hl : n1 - 1;
     const uint16_t* qn = reinterpret_cast<const uint16_t*>(a.q) + ((int64_t)r * n1 + hc) * D + (lane >> 5) * 8;
     const uint16_t* qrr = reinterpret_cast<const uint16_t*>(a.qr) + ((int64_t)r * n1 + hc) * DR + (lane >> 5) * 8;
 #pragma unroll
@@ -1940,14 +1938,13 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
   if (ntok == 0) {
     wait_vmcnt<0>();
-    if (ntok_all == 0 && sp == 0) {   // skipped row: zeros (out, stats) for this half's heads
-      const int hn = n1 - h0 < w8::HH ? n1 - h0 : w8::HH;
-      for (int i = tid; i < hn * D / 8; i += w8::NW * 64)
-        stg16(out + ((int64_t)r * n1 + h0) * D + i * 8, make_uint4(0, 0, 0, 0));
+    if (ntok_all == 0 && sp == 0) {   // skipped row: zeros (out, stats)
+      for (int i = tid; i < n1 * D / 8; i += w8::NW * 64)
+        stg16(out + (int64_t)r * n1 * D + i * 8, make_uint4(0, 0, 0, 0));
       if (a.sm_max)
-        for (int h = tid; h < hn; h += w8::NW * 64) {
-          a.sm_max[(int64_t)r * n1 + h0 + h] = 0.f;
-          a.sm_sum[(int64_t)r * n1 + h0 + h] = 0.f;
+        for (int h = tid; h < n1; h += w8::NW * 64) {
+          a.sm_max[(int64_t)r * n1 + h] = 0.f;
+          a.sm_sum[(int64_t)r * n1 + h] = 0.f;
         }
     }
     return;
@@ -1993,7 +1990,7 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
 #pragma unroll
   for (int t = 0; t < 4; ++t) ids_dma(t);
   wait_vmcnt<0>();
-  if (hs >= n1)
+  if (hl >= n1)
 #pragma unroll
     for (int j = 0; j < w8::KQ; ++j) qf[j] = make_uint4(0, 0, 0, 0);
   if (tid < 2) s_flag[tid] = 0;
@@ -2211,15 +2208,15 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
     }
     inv[mt] = 1.f / lt;   // l > 0: a row or split holds at least one token
     // statistics: wave (hb = mt, kq = 0) holds m_used of these heads
-    if (kq == 0 && hb == mt && lane < 32 && h0 + h < n1) {
-      const int64_t hr = (int64_t)r * n1 + h0 + h;
+    if (kq == 0 && hb == mt && lane < 32 && h < n1) {
+      const int64_t hr = (int64_t)r * n1 + h;
       if (direct) {
         if (a.sm_max) {
           a.sm_max[hr] = mtr;
           a.sm_sum[hr] = lt * exp2f((m_used - mtr) * LOG2E);
         }
       } else {
-        float* ps = ws.part_s + (((int64_t)r * splits + sp) * n1 + h0 + h) * 3;
+        float* ps = ws.part_s + (((int64_t)r * splits + sp) * n1 + h) * 3;
         ps[0] = m_used;
         ps[1] = mtr;
         ps[2] = lt;
@@ -2231,7 +2228,7 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   // leave 16-byte runs (as in the 128-head form)
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
-    const int ha = h0 + mt * 32 + (lane & 31);
+    const int ha = mt * 32 + (lane & 31);
     const int hc = ha < n1 ? ha : n1 - 1;
     uint16_t* orow = (direct ? out + ((int64_t)r * n1 + hc) * D
                              : ws.part_o + (((int64_t)r * splits + sp) * n1 + hc) * D) +
