@@ -46,6 +46,7 @@
 // Unlike the reference (sparse_flash_attention_triton.py:509-525) the fp32
 // accumulator never round-trips through HBM for unsplit rows.
 #include <climits>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -1864,7 +1865,7 @@ void sfa_attn2_kernel(SfaArgs a, int splits, Ws ws) {
 
 // ---------------------------------------------------------------- kernel 2, 64-head form (D = 512)
 // One work-group of 8 waves (two per SIMD) per (query row, 64 heads, KV split), launched
-// for N1 <= 64 where the work-groups number at most one a CU (see launch_attn_d). O^T and Q^T of 64 heads take half the
+// for N1 <= 64 where the rows have a CU each (see two_wave_form). O^T and Q^T of 64 heads take half the
 // registers of the 128-head form, so two waves share each SIMD.
 //  * S^T[32 tokens, 32 heads] of head block hb = w % 2 is split over the contraction:
 //    wave w runs k-steps [9 q, 9 q + 9), q = w / 2 (Q^T fragments of those k-steps, rope
@@ -2254,16 +2255,57 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
   }
 }
 
+// The two-wave form (two rows a CU) or the eight-wave one (a row a CU). At most 256 work-groups: the latter.
+// More than 512: the former (at no size slower by more than 1%). Between, rows of equal length would make
+// the eight-wave form take two rounds, but rows of a short causal prompt do not: the longest come first and the
+// short ones fill the gaps. So both are estimated from the row lengths, in tokens of the eight-wave form
+// (59 ns), where a row costs F besides its own:
+//  * eight waves: the longest row; all of them over 256 CUs; or two of the shortest;
+//  * two waves: a pair on one CU runs at 1 / 1.2 of that speed each, a row alone at 1 / 1.33; the first pair is row 0
+//    and row 256.
+// 300 causal rows of one prompt 26.1 us with eight waves, 33.1 with two; 512 rows 39.0 | 43.5; 257 rows after
+// 200 keys 35.3 | 40.6, after 500 59 | 56; 300 rows after 1500, 2048 tokens, 150 | 119. Over 672 such calls (257 .. 512
+// rows, 1 .. 16 prompts, 16 and 64 heads) the choice is within 5% of the faster one, always-two-waves within 27%.
+// Lengths are known here as the longest key length (s2) and, for contiguous keys, the keys and rows in all: the
+// prompts but the longest are taken as equal.
+inline bool two_wave_form(const SfaArgs& a, int cap, int splits) {
+  const int64_t nq = (int64_t)a.total_rows * splits;
+  if (nq <= 256) return false;
+  if (nq > 512 || splits > 1 || a.sparse_mode == 0 || a.batch <= 0) return true;
+  constexpr float F = 224.f, OVERLAP = 0.88f, PAIR = 1.2f, ALONE = 1.33f;
+  const int rows = a.total_rows;
+  // keys before a prompt's first row: paged, the pool says nothing about the lengths in use (as long as they may be)
+  const int mean_rows = (rows + a.batch - 1) / a.batch;
+  const int64_t mean_keys = a.block_table ? a.s2 : a.key_rows / a.batch;
+  const int past = (int)(mean_keys > mean_rows ? (mean_keys - mean_rows < a.s2 ? mean_keys - mean_rows : a.s2) : 0);
+  int n = a.s2 - past;   // rows of the longest prompt
+  n = n < 1 ? 1 : (n < rows ? n : rows);
+  const int rest = a.batch > 1 ? (rows - n) / (a.batch - 1) : 0;
+  auto len = [&](int64_t keys) { return (float)(keys < 1 ? 1 : (keys < cap ? keys : cap)); };
+  // tokens of m rows that see past + 1 .. past + m keys
+  auto ramp = [&](int m) {
+    const int full = past + m > cap ? (past + m - cap < m ? past + m - cap : m) : 0, part = m - full;
+    return (float)full * cap + (float)part * (past + 0.5f * (part + 1));
+  };
+  const float longest = len(past + n), shortest = len(past + 1);
+  const float tokens = ramp(n) + (a.batch - 1) * ramp(rest);
+  const float eight = fmaxf(F + longest, fmaxf((tokens + F * OVERLAP * rows) / 256, 2 * (shortest + F * OVERLAP)));
+  const int m = 256 % n;   // row 256 lies m rows before the end of its prompt
+  float second = len(past + n - m);
+  if (rows > 256 + n - m) second = fmaxf(second, len(past + m));
+  return PAIR * (F + second) + ALONE * (longest - second) <= eight;
+}
+
 template <int IO, int D>
 hipError_t launch_attn_d(const SfaArgs& a, hipStream_t s, int cap, int splits, int fuse_tok, Ws ws) {
   // Both per-wave forms gather with 32-bit row offsets. With N1 <= 64, D = 512 and token lists from
   // the token-list launch: the two-wave form, whose work-groups share a CU by twos (4026 packed rows of
-  // 64 heads, fp16, 808 -> 585 us; 32 heads 763 -> 523; 300 rows of 2048 tokens 206 -> 145), unless there is
-  // at most one a CU: then eight waves on a row (256 rows 124 us against 154). Above 64 heads one
-  // work-group of four waves per row: two of the two-wave form would gather every row twice.
+  // 64 heads, fp16, 808 -> 585 us; 32 heads 763 -> 523; 300 rows of 2048 tokens 206 -> 145), unless a row
+  // has a CU to itself (two_wave_form): then eight waves on a row (256 rows 124 us against 154). Above 64
+  // heads one work-group of four waves per row: two of the two-wave form would gather every row twice.
   const bool off32 = (uint64_t)a.key_rows * D * 2 <= (1ull << 32);
   const int64_t nq = (int64_t)a.total_rows * splits;
-  if (D == w2::D && !fuse_tok && a.n1 <= w2::NW * 32 && off32 && nq > 256) {
+  if (D == w2::D && !fuse_tok && a.n1 <= w2::NW * 32 && off32 && two_wave_form(a, cap, splits)) {
     hipLaunchKernelGGL(sfa_attn2_kernel<IO>, dim3(a.total_rows, splits), dim3(w2::NW * 64), 0, s, a, splits, ws);
   } else if (D == w8::DD && !fuse_tok && a.n1 <= w8::HH) {
     hipLaunchKernelGGL(sfa_attn8_kernel<IO>, dim3((unsigned)nq), dim3(w8::NW * 64), 0, s, a, splits, ws);

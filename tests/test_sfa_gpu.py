@@ -532,6 +532,29 @@ def test_two_wave_form_rows_of_every_length(dev, N1, dtype, scale):
     compare(out, smax, ssum, *o, what=f"two-wave N1={N1} {dtype} scale={scale}")
 
 
+@pytest.mark.parametrize("N1,dtype", [(16, "fp16"), (64, "bf16")])
+@pytest.mark.parametrize("lens,past", [((270,), 0), ((400,), 90), ((150, 128), 0), ((30, 300), 0)])
+def test_short_causal_prompts_between_the_forms(dev, lens, past, N1, dtype):
+    """257 .. 512 packed rows of short causal prompts, on both sides of the line between the eight-wave
+    form and the two-wave one: every row length from one token on."""
+    D, T, count = 512, sum(lens), max(lens) + past
+    kv = [n + past for n in lens]
+    rng = np.random.RandomState(26)
+    t = lambda *s: torch.from_numpy(rng.randn(*s).astype(np.float32)).to(DT[dtype])
+    q, qr, k, kr = t(T, N1, D), t(T, N1, 64), t(sum(kv), 1, D), t(sum(kv), 1, 64)
+    si = np.full((T, 1, count), -1, np.int32)
+    for r, n in enumerate(past + 1 + i for m in lens for i in range(m)):
+        si[r, 0, :n] = rng.permutation(n)
+    kw = dict(scale_value=0.04, actual_seq_lengths_query=np.cumsum(lens).tolist(),
+              actual_seq_lengths_kv=np.cumsum(kv).tolist(), layout_query="TND", layout_kv="TND", sparse_mode=3,
+              return_softmax_lse=True)
+    out, smax, ssum = sparse_flash_attention(q.to(dev), k.to(dev), k.to(dev), torch.from_numpy(si).to(dev),
+                                             query_rope=qr.to(dev), key_rope=kr.to(dev), **kw)
+    torch.cuda.synchronize()
+    o = SFA.sparse_flash_attention(_np(q), _np(k), None, si, query_rope=_np(qr), key_rope=_np(kr), io_dtype=dtype, **kw)
+    compare(out, smax, ssum, *o, what=f"short prompts {lens} after {past}, N1={N1} {dtype}")
+
+
 @pytest.mark.parametrize("N1,dtype", [(16, "bf16"), (64, "fp16")])
 @pytest.mark.parametrize("S1,S2,kv_splits", [(140, 140, 2), (60, 200, 5)])
 def test_two_wave_form_split_partials(dev, N1, dtype, S1, S2, kv_splits):
