@@ -338,3 +338,28 @@ def test_grad_64_head_rows(dev, N1, dtype):
     torch.cuda.synchronize()
     for name, a, b in zip(("dq", "dk", "dv", "dqr", "dkr"), again, got):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"N1={N1}: {name} differs"
+
+
+@pytest.mark.parametrize("N1", [32, 64])
+def test_grad_tokens_past_the_keys(dev, N1):
+    """act_k past the key tensor (180 of 140 keys): the selected tokens past it read as zero rows (32
+    heads: the 32-head rows kernel, 64: the 64-head one). The oracle gets those rows as zeros; its
+    gradients of the keys that exist are the call's."""
+    S1, S2, past, count, D, dtype = 140, 140, 40, 70, 512, "bf16"
+    q, k, _, qr, kr, do = _inputs(1, S1, S2, N1, D, dtype)
+    si = _ref_indices(1, S1, S2 + past, count, 1, 3)
+    assert (si >= S2).sum() > 50
+    scale = 1.0 / math.sqrt(D + 64)
+    g = lambda x: x.to(dev)
+    kw = dict(scale_value=scale, actual_seq_lengths_kv=[S2 + past], query_rope=g(qr), key_rope=g(kr), sparse_mode=3)
+    ids = g(torch.from_numpy(si))
+    out, smax, ssum = sparse_flash_attention(g(q), g(k), g(k), ids, return_softmax_lse=True, **kw)
+    got = sparse_flash_attention_grad(g(q), g(k), g(k), ids, g(do), out, smax, ssum, **kw)
+    torch.cuda.synchronize()
+    pad = lambda x: np.concatenate([_np(x), np.zeros((1, past) + tuple(x.shape[2:]), np.float32)], axis=1)
+    want = list(SFG.sparse_flash_attention_grad(_np(q), pad(k), None, si, _np(do), _np(out), _np(smax), _np(ssum),
+                                                scale, _np(qr), pad(kr), None, [S2 + past], 1, "BSND", 3,
+                                                io_dtype=dtype))
+    for i in (1, 2, 4):
+        want[i] = want[i][:, :S2]
+    _check(got, want, dtype, S1, f"tokens past the keys N1={N1}")
