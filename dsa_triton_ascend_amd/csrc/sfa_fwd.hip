@@ -2485,7 +2485,11 @@ __global__ __launch_bounds__(256, 2) void sfa_teach64_kernel(SfaArgs a, Ws ws) {
 template <int IO, int D>
 hipError_t launch_teach_d(const SfaArgs& a, hipStream_t s, int cap, Ws ws) {
   if constexpr (D == w2::D) {
-    if (a.n1 <= 64 && (uint64_t)a.key_rows * D * 2 <= (1ull << 32)) {   // 32-bit row offsets
+    // 32-bit row offsets; and not few short rows of 33 .. 64 heads, where its prologue (every lane loads Q itself)
+    // costs more than its tiles save: the sparse loss of 64 rows with 16 slots 45.6 us in the form below, 47.7 here,
+    // with 256 slots 66.1 | 66.5, with 512 90.1 | 88.8; of 512 rows with 64 99.2 | 98.1
+    const bool few_short = a.n1 > 32 && a.total_rows <= 256 && cap < 256;
+    if (a.n1 <= 64 && !few_short && (uint64_t)a.key_rows * D * 2 <= (1ull << 32)) {
       hipLaunchKernelGGL(sfa_teach64_kernel<IO>, dim3(a.total_rows), dim3(256), 0, s, a, ws);
       return hipGetLastError();
     }

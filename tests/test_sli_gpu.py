@@ -255,6 +255,14 @@ def test_kl_loss_fp32_weights(dev, dtype):
 
 @pytest.mark.parametrize("N1,dtype", [(64, "bf16"), (32, "fp16")])
 def test_kl_loss_teacher_rows_of_every_length(dev, N1, dtype):
-    """D = 512 with at most 64 heads (the 64-head teacher): 70 rows of 1 .. 70 slots, every remainder
-    of its 32-slot tiles and 16-slot halves, and a second batch of shorter lengths."""
+    """D = 512 with at most 64 heads (the 64-head teacher; at 64 heads the one it replaces takes so few
+    short rows): 70 rows of 1 .. 70 slots, every remainder of its 32-slot tiles and 16-slot halves, and a
+    second batch of shorter lengths."""
     run(dev, 2, 70, 70, N1, 512, 64, 128, 70, dtype, "causal_random", act_q=[70, 40], act_k=[70, 45], loose=True)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_kl_loss_64_head_teacher_short_rows(dev, dtype):
+    """The same rows in four batches: more than 256 rows, which the 64-head teacher takes at any length."""
+    run(dev, 4, 70, 70, 64, 512, 64, 128, 70, dtype, "causal_random", act_q=[70, 40, 70, 1],
+        act_k=[70, 45, 69, 70], loose=True)
