@@ -371,6 +371,22 @@ def pmc_pass(torch, W):
              scale_value=g.scale_value, query_rope=g.query_rope, key_rope=g.key_rope,
              sparse_mode=g.sparse_mode).run()
     torch.cuda.synchronize()
+    from dsa_triton_ascend_amd.sli_grad_kl_loss import KLLossPlan
+    gen = torch.Generator(device=dev).manual_seed(5)
+    randn = lambda *shape: torch.randn(shape, device=dev, generator=gen).to(torch.bfloat16)
+    KLLossPlan(g.query, g.key, randn(1, 512, 64, 128), randn(1, 4096, 1, 128), randn(1, 512, 64), g.sparse_indices,
+               smax, ssum, query_rope=g.query_rope, key_rope=g.key_rope, scale_value=g.scale_value).run()
+    torch.cuda.synchronize()
+    del g, out, smax, ssum
+    # one decode step of the indexer: 64 sequences of 4K to 32K keys, pages of 64, each in place
+    lens = [4096 + 28672 * (2 * (37 * b % 64) + 1) // 128 for b in range(64)]
+    pages = [(n + 63) // 64 for n in lens]
+    table = torch.full((64, max(pages)), -1, dtype=torch.int32)
+    for b, n in enumerate(pages):
+        table[b, :n] = torch.arange(n) + sum(pages[:b])
+    IndexerPlan(randn(64, 1, 64, 128), randn(sum(pages), 64, 1, 128), randn(64, 1, 64), None, lens, table.to(dev),
+                layout_key="PA_BSND", sparse_count=2048, sparse_mode=3).run()
+    torch.cuda.synchronize()
     log("[pmc-pass] done")
 
 
@@ -394,8 +410,8 @@ def main():
     ap.add_argument("--quick", action="store_true", help="headline only (no breakdown, no CPU baseline)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--pmc-pass", action="store_true",
-                    help="for rocprofv3 --pmc: one C2 indexer call, one SFA prefill/decode call and a "
-                         "512 MiB plain copy (the counter calibration), no timing")
+                    help="for rocprofv3 --pmc: a 512 MiB plain copy (the counter calibration) and one call each of "
+                         "the indexer, attention, its backward and the sparse loss, no timing")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU: this build has no multi-GPU path (asked for --gpus {args.gpus}); "
