@@ -139,7 +139,7 @@ struct BatchGeo {
 __host__ __device__ inline int batch_nk(int act_k, int s2) { return act_k < 0 ? 0 : (act_k < s2 ? act_k : s2); }
 
 // (64 more where the row would be a multiple of 2 KiB: dense rows a power of two apart put a product's
-// column panel on few memory channels; 512 rows of 64 heads over 4096 keys 740 -> 719 us the call)
+// column panel on few memory channels; 3% of the call at 512 rows of 64 heads over 4096 keys)
 __host__ __device__ inline int dense_row(int nq, int n1) {
   const int r = (nq * n1 + GBK - 1) / GBK * GBK;
   return r % 1024 == 0 ? r + GBK : r;
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(BWV * 64) void sfa_bwd_rows_kernel(SfaBwdArgs a, Sf
 //  * P and dS also pass through a 2.5 KB LDS tile of the wave's own, from which transposed reads give each
 //    lane four heads of one token for the dense buffers' stores.
 // 512 rows of 64 heads over 4096 keys, 2048 tokens a row: this kernel 370 us against 560 for the 32-head
-// form (968 -> 719 us the call). Without its stores and gathers it takes 211 us, of which 101 of MFMA
+// form (949 -> 725 us the call). Without its stores and gathers it takes 211 us, of which 101 of MFMA
 // at one wave per SIMD; the 536 MB of P, dS and zeros, in runs of 32 to 128 bytes, cost the rest.
 namespace r64 {
 constexpr int D = 512, DT = D + BDR;
@@ -793,7 +793,7 @@ void sfa_bwd_rows64_kernel(SfaBwdArgs a, SfaTokenLists tl, BwdWs w) {
       // this wave's gathers of tile t. The GPW loads of the tile after it were issued later, so at most GPW
       // operations left means that these have landed; stores retire out of order with loads, so none
       // is counted on (a wait that counted them read rows that had not landed). Two tiles ahead, the
-      // wait leaves room for the last tile's stores; one tile ahead it waited for them (743 us the call).
+      // wait leaves room for the last tile's stores; one tile ahead it waited for them (3% of the call).
       if (t == 0) wait_vmcnt<GPW - 1>(); else wait_vmcnt<GPW>();
       if (zr0) {   // rare: rows out of range read as zeros
         wait_vmcnt<0>();

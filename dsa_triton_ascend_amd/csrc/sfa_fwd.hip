@@ -1473,9 +1473,10 @@ __global__ __launch_bounds__(NWV * 64) void sfa_attn_kernel(SfaArgs a, int cap, 
 // S^T, the softmax and PV of its own 32 heads over all columns, P in its registers. Two work-groups
 // share a CU (one wave per SIMD each: O^T takes 256 AGPRs, Q^T with its rope 144 VGPRs), so a CU
 // works on two query rows at once and one row's prologue and epilogue run beside the other's tiles.
-// A pair of tiles takes about 4,650 cycles against 2,176 of MFMA, the same as the 128-head form (and
-// without its gathers, 15%, the chip's clock under this load is most of what is left); the eight-wave
-// form this replaces took 3,600 per single tile.
+// A pair of tiles takes about 4,600 cycles, 2,176 of them of MFMA (47%; the 128-head form 55%); the
+// eight-wave form this replaces took 3,600 per single tile. By the counters (512 rows of 2048 tokens) a
+// wave issues for 47% of its life, waits for data or the barrier for 26% and to issue for 27%; without
+// its gathers the call takes 15% less.
 //  * The ring holds two 32-token tiles (two work-groups' rings fill the LDS): the gathers of tile t+1
 //    ride on the S^T chain of tile t and have its softmax and PV to land. One barrier per tile.
 //  * Rows are unpadded (1024 B), their chunks permuted by kv_swz.
