@@ -663,22 +663,28 @@ void launch_mt(const LiScoreArgs& a, hipStream_t s, int MT, dim3 grid, dim3 bloc
 // Number of work-groups over which a row block's keys are split (tiles of bn keys), so that few row
 // blocks fill the chip: the split with the shortest modelled time. Only max_kv is known here.
 //  * Q in registers (qreg): one work-group a CU; each costs about 10 tiles of 64 keys besides its own (Q,
-//    the first tiles' latency). The time is at least the longest work-group's, the mean work's over 256
+//    the first tiles' latency), 2 with little Q (64 wide, at most 32 heads: 3 x 700 rows of 1500 keys, 264
+//    row blocks, 20.5 us whole, 17.2 in 2 or 3). The time is at least the longest work-group's, the mean work's over 256
 //    CUs, and that of whole rounds of the shortest ones (under a causal mask the row blocks see between
 //    max_kv - rows and max_kv keys). With several sequences 3 parts of 10 go to the case that they hold
 //    half of max_kv on average and later work-groups fill the gaps.
 //  * Q read from L2 again for every tile (more than 64 heads a key head): a split costs half a tile, and ten
-//    or more keep a work-group's keys small enough for its XCD's L2.
+//    or more keep a work-group's keys small enough for its XCD's L2. Not where the Q of an XCD's 32
+//    work-groups stays in its 4 MiB (few rows a batch; 100 x 1 row of 700 keys, 64 wide, 25.6 us in 2,
+//    33.4 in 10) or the keys are so few that Q is hardly read again (40 x 30 rows of 300 keys 43.0 whole,
+//    51.3 in 5): then a split costs one tile.
 // Against at most 16 splits towards 512 work-groups: 512 rows of 4096 keys 37.7 -> 31.0 us (4 splits), 64 of
 // 16000 26.1 -> 18.4 (32), 8 of 100000, one sequence, 75 -> 11.2 (256); paged, 64 sequences of 4096, 5 rows,
 // 38.8 -> 32.7 (4), 100 of 3000, 8 rows, 61.1 -> 47.5 (2); 128 heads, 512 rows of 4096 798 -> 279 (16).
-inline int key_split(const LiScoreArgs& a, int bn, bool qreg) {
+inline int key_split(const LiScoreArgs& a, int bn, bool qreg, bool small_q) {
   const int64_t blocks = (int64_t)((a.max_rows_per_batch + NW - 1) / NW) * a.n2 * a.batch;
   const int tiles = a.max_kv > 0 ? (a.max_kv - 1) / bn + 1 : 0;
   const int cap = qreg || blocks == 0 ? 256 : (int)(blocks < 8 ? 256 / blocks : 32);
   const int most = tiles < cap ? tiles : cap;
-  const int least = qreg ? 1 : (tiles < 10 ? tiles : 10);
-  const float over = qreg ? (bn > 64 ? 5.f : 10.f) : 0.5f;
+  const int64_t live_q = (int64_t)32 * (a.max_rows_per_batch < NW ? a.max_rows_per_batch : NW) * (a.n1 / a.n2) * a.d * 2;
+  const bool reread = !qreg && live_q >= (4 << 20) && (tiles > 6 || blocks > 256);
+  const int least = !reread ? 1 : (tiles < 10 ? tiles : 10);
+  const float over = qreg ? (small_q ? 2.f : (bn > 64 ? 5.f : 10.f)) : (reread ? 0.5f : 1.f);
   const int hidden = a.sparse_mode == 3 ? (a.max_rows_per_batch < a.max_kv ? a.max_rows_per_batch : a.max_kv) : 0;
   const float shortest = qreg ? (float)(a.max_kv - hidden) / bn : (float)tiles, mean = (tiles + shortest) / 2;
   float best = INFINITY;
@@ -707,7 +713,7 @@ hipError_t launch_d(const LiScoreArgs& a0, hipStream_t s, int MT) {
     else launch_rows<IO, false>(a, s, MT);
     return hipGetLastError();
   }
-  a.key_split = key_split(a, LiTile<D>::BN, MT <= 2 && MT * D <= 512);
+  a.key_split = key_split(a, LiTile<D>::BN, MT <= 2 && MT * D <= 512, MT * D <= 64);
   dim3 grid((unsigned)(((a.max_rows_per_batch + NW - 1) / NW) * a.key_split), a.n2, a.batch), block(NW * 64);
   if (a.block_table)
     launch_mt<IO, D, true>(a, s, MT, grid, block);
