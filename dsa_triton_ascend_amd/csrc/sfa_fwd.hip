@@ -2268,12 +2268,15 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
 // 200 keys 35.3 | 40.6, after 500 59 | 56; 300 rows after 1500, 2048 tokens, 150 | 119. Over 672 such calls (257 .. 512
 // rows, 1 .. 16 prompts, 16 and 64 heads) the choice is within 5% of the faster one, always-two-waves within 27%.
 // Lengths are known here as the longest key length (s2) and, for contiguous keys, the keys and rows in all: the
-// prompts but the longest are taken as equal.
+// prompts but the longest are taken as equal. (Forced) KV splits are work-groups of shorter rows: the launch
+// takes all rows' first splits, then all rows' second ones.
 inline bool two_wave_form(const SfaArgs& a, int cap, int splits) {
   const int64_t nq = (int64_t)a.total_rows * splits;
   if (nq <= 256) return false;
-  if (nq > 512 || splits > 1 || a.sparse_mode == 0 || a.batch <= 0) return true;
-  constexpr float F = 224.f, OVERLAP = 0.88f, PAIR = 1.2f, ALONE = 1.33f;
+  if (nq > 512 || a.sparse_mode == 0 || a.batch <= 0) return true;
+  // LATE: with KV splits the two-wave form asks for its token ids only after the row's count (130 causal rows
+  // in two splits 18.9 us with eight waves, 22.1 with two; after 3000 keys, 512 tokens, 44.1 | 35.7)
+  constexpr float F = 224.f, OVERLAP = 0.88f, PAIR = 1.2f, ALONE = 1.33f, LATE = 120.f;
   const int rows = a.total_rows;
   // keys before a prompt's first row: paged, the pool says nothing about the lengths in use (as long as they may be)
   const int mean_rows = (rows + a.batch - 1) / a.batch;
@@ -2282,7 +2285,7 @@ inline bool two_wave_form(const SfaArgs& a, int cap, int splits) {
   int n = a.s2 - past;   // rows of the longest prompt
   n = n < 1 ? 1 : (n < rows ? n : rows);
   const int rest = a.batch > 1 ? (rows - n) / (a.batch - 1) : 0;
-  auto len = [&](int64_t keys) { return (float)(keys < 1 ? 1 : (keys < cap ? keys : cap)); };
+  auto len = [&](int64_t keys) { return (float)(keys < 1 ? 1 : (keys < cap ? keys : cap)) / splits; };
   // tokens of m rows that see past + 1 .. past + m keys
   auto ramp = [&](int m) {
     const int full = past + m > cap ? (past + m - cap < m ? past + m - cap : m) : 0, part = m - full;
@@ -2290,11 +2293,11 @@ inline bool two_wave_form(const SfaArgs& a, int cap, int splits) {
   };
   const float longest = len(past + n), shortest = len(past + 1);
   const float tokens = ramp(n) + (a.batch - 1) * ramp(rest);
-  const float eight = fmaxf(F + longest, fmaxf((tokens + F * OVERLAP * rows) / 256, 2 * (shortest + F * OVERLAP)));
+  const float eight = fmaxf(F + longest, fmaxf((tokens + F * OVERLAP * nq) / 256, 2 * (shortest + F * OVERLAP)));
   const int m = 256 % n;   // row 256 lies m rows before the end of its prompt
   float second = len(past + n - m);
-  if (rows > 256 + n - m) second = fmaxf(second, len(past + m));
-  return PAIR * (F + second) + ALONE * (longest - second) <= eight;
+  if (nq > 256 + n - m) second = fmaxf(second, len(past + m));
+  return PAIR * (F + second) + ALONE * (longest - second) + (splits > 1 ? LATE : 0.f) <= eight;
 }
 
 template <int IO, int D>

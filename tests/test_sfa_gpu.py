@@ -556,12 +556,12 @@ def test_short_causal_prompts_between_the_forms(dev, lens, past, N1, dtype):
 
 
 @pytest.mark.parametrize("N1,dtype", [(16, "bf16"), (64, "fp16")])
-@pytest.mark.parametrize("S1,S2,kv_splits", [(140, 140, 2), (60, 200, 5)])
+@pytest.mark.parametrize("S1,S2,kv_splits", [(300, 300, 2), (60, 200, 5), (140, 140, 2)])
 def test_two_wave_form_split_partials(dev, N1, dtype, S1, S2, kv_splits):
     """The two-wave form on KV splits (forced; sparse_block_size 2, so the token lists come from their
     launch; more than 256 work-groups): partials and statistics of the splits that hold tokens, rows so
     short that one split holds all (it writes the output itself) or the later ones are empty, and a
-    row without tokens."""
+    row without tokens. (140 short rows in two splits go to the eight-wave form.)"""
     B, D, count, bs = 1, 512, S2 // 2, 2
     assert S1 * kv_splits > 256
     q, k, _, qr, kr = _inputs(B, S1, S2, N1, D, dtype, seed=24)
