@@ -2266,7 +2266,7 @@ __global__ __launch_bounds__(w8::NW * 64) void sfa_attn8_kernel(SfaArgs a, int s
 //    and row 256.
 // 300 causal rows of one prompt 26.1 us with eight waves, 33.1 with two; 512 rows 39.0 | 43.5; 257 rows after
 // 200 keys 35.3 | 40.6, after 500 59 | 56; 300 rows after 1500, 2048 tokens, 150 | 119. Over 672 such calls (257 .. 512
-// rows, 1 .. 16 prompts, 16 and 64 heads) the choice is within 5% of the faster one, always-two-waves within 27%.
+// rows, 1 .. 16 prompts, 16 and 64 heads) the choice is within 7% of the faster one, always-two-waves within 27%.
 // Lengths are known here as the longest key length (s2) and, for contiguous keys, the keys and rows in all: the
 // prompts but the longest are taken as equal. (Forced) KV splits are work-groups of shorter rows: the launch
 // takes all rows' first splits, then all rows' second ones.
