@@ -628,8 +628,9 @@ inline RowsShape rows_shape(const LiScoreArgs& a) {
   return {chunk, nchunk, ((int64_t)nchunk * a.batch + 7) / 8 * 8 * a.max_rows_per_batch};
 }
 
-// Whether the few-row kernel takes the call. One row a batch: always (it was the faster one at each of
-// 1 .. 1000 sequences of 128 .. 100000 keys, by 5% to 9x). Two rows: where a sequence has more than a
+// Whether the few-row kernel takes the call. One row a batch: always (the faster one, by 5% to 9x, of 1 .. 1000
+// sequences of 128 .. 100000 keys, but where equal lengths end just past a round: 16 of 9000 keys, contiguous,
+// 14.3 us against 12.7; a chunk that suits them, 512 keys 11.5, makes uneven ones slower, 11.4 against 9.6). Two rows: where a sequence has more than a
 // few subtiles, else its second work-group costs more than the shared read saves (512 sequences of
 // 128 keys 11.6 us in the kernel above, 13.5 here; 256 of 500 12.0 against 11.3), and, on contiguous keys,
 // up to 400 MB of them (512 of 4096, 537 MB: 122.6 against 130.7; 256 of 6000, 393 MB: 96.7 against 94.2;
